@@ -58,6 +58,42 @@ __device__ __forceinline__ void rope_rotate(uint16_t x, uint16_t y, float c, flo
 // 2^x on v_exp_f32 (1 ulp; flushes below 2^-126, 2^-inf = 0).
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// ---- global memory -> LDS without registers ---------------------------------
+// global_load_lds_dwordx4: lane l of the wave writes the 16 bytes it fetches to
+// LDS address `lds` + 16 l (`lds` wave-uniform, in M0). Written as inline asm
+// because the compiler counts the builtin's LDS write against every later
+// ds_read of the workgroup's LDS and waits vmcnt(0) before the first one: a
+// tile prefetched into the other buffer was waited for before the current
+// tile's first operand read (a 16k-token prompt's causal attention 1725 us, with
+// the asm 1619; five 512-token chunks through a paged pool, with their
+// projection, 623 and 593). The asm has no output register and its address
+// registers are read when it issues; the caller waits (lds_dma_wait, then a
+// barrier) before anything reads the tile. M0 is a reserved register that no
+// other instruction of these kernels uses.
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return __builtin_amdgcn_readfirstlane(
+        uint32_t(uintptr_t((__attribute__((address_space(3))) const char*)p)));
+}
+__device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds),
+                 "v"(src)
+                 : "memory");
+}
+// The same from a wave-uniform base plus a per-lane 32-bit offset.
+__device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds),
+                 "v"(off), "s"(base)
+                 : "memory");
+}
+
+// Waits for the wave's vector-memory operations, the DMA above among them (the
+// builtin, so that the compiler also knows its own loads have arrived).
+__device__ __forceinline__ void lds_dma_wait() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), other counters free
+    asm volatile("" ::: "memory");
+}
+
 // ---- cross-lane reductions (wave64) -----------------------------------------
 // DPP move of v (row_mask, bank_mask all lanes; bound_ctrl: a source lane
 // outside the row would read 0, which none of the controls used here has).

@@ -169,39 +169,39 @@ __device__ __forceinline__ uint4 ld16(const uint16_t* p) {
 template <bool IS_K, bool PAGED>
 __device__ __forceinline__ void dma_tile(const char* base, uint32_t row_bytes, int key0,
                                          int kv_len, int wave, int lane, char* lds_tile,
-                                         const int (&blk)[4], int bs_log2) {
+                                         const int (&blk)[4], int bs_log2, int max_block) {
     const int pr = lane >> 4, pc = lane & 15;
+    const uint32_t dst = lds_address(lds_tile) + 16 * wave * 256;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int r = 16 * wave + 4 * i + pr;  // tile row
         const int chunk = IS_K ? (pc ^ (r & 15)) : (pc ^ (4 * (r & 3)));
         const int key = min(key0 + r, kv_len - 1);
-        const char* src;
         if constexpr (PAGED) {
-            const int64_t slot = (int64_t(blk[i]) << bs_log2) | (key & ((1 << bs_log2) - 1));
-            src = base + slot * row_bytes + 16 * chunk;
+            const int b = min(max(blk[i], 0), max_block);  // never address outside the pool
+            const int64_t slot = (int64_t(b) << bs_log2) | (key & ((1 << bs_log2) - 1));
+            lds_dma16(base + slot * row_bytes + 16 * chunk, dst + 4 * i * 256);
         } else {
-            src = base + (__umul24(uint32_t(key), row_bytes) + 16u * chunk);
+            lds_dma16(base, __umul24(uint32_t(key), row_bytes) + 16u * chunk, dst + 4 * i * 256);
         }
-        __builtin_amdgcn_global_load_lds(
-            src, (__attribute__((address_space(3))) void*)(lds_tile + (16 * wave + 4 * i) * 256),
-            16, 0, 0);
     }
 }
 
-// Physical blocks of the rows this lane fetches for tile `kt` (paged pools).
-__device__ __forceinline__ void tile_blocks(const int32_t* table, int bs_log2, int max_block, int kt,
-                                            int kv_len, int wave, int lane, int (&blk)[4]) {
+// Block-table entries of the rows this lane fetches for tile `kt` (paged pools),
+// as loaded: dma_tile clamps them to the pool when it uses them, a tile later.
+// (Clamped here, the wait for the entries would also wait for the tile DMA
+// issued just before them.)
+__device__ __forceinline__ void tile_blocks(const int32_t* table, int bs_log2, int kt, int kv_len,
+                                            int wave, int lane, int (&blk)[4]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int key = min(kt * kPfKeys + 16 * wave + 4 * i + (lane >> 4), kv_len - 1);
-        blk[i] = min(max(table[key >> bs_log2], 0), max_block);  // never address outside the pool
-    }
+    for (int i = 0; i < 4; ++i)
+        blk[i] = table[min(kt * kPfKeys + 16 * wave + 4 * i + (lane >> 4), kv_len - 1) >> bs_log2];
 }
 
-// Physical block of logical row `key` (paged pools), clamped to the pool.
-__device__ __forceinline__ int table_block(const PrefillArgs& a, int key) {
-    return min(max(a.table[key >> a.bs_log2], 0), a.max_block);
+// Block-table entry of logical row `key` (paged FP8 pools), as loaded: fp8_load
+// clamps it to the pool a tile later, for the same reason.
+__device__ __forceinline__ int table_entry(const PrefillArgs& a, int key) {
+    return a.table[key >> a.bs_log2];
 }
 
 // FP8 pools: tile rows go through registers, 32 codes of K and of V per thread
@@ -216,10 +216,11 @@ struct Fp8Tile {
 template <bool PAGED>
 __device__ __forceinline__ void fp8_load(const char* kb, const char* vb, uint32_t row_bytes,
                                          int key0, int kv_len, int tid, int blk, int bs_log2,
-                                         Fp8Tile& t) {
+                                         int max_block, Fp8Tile& t) {
     const int key = min(key0 + (tid >> 2), kv_len - 1);
+    const int b = min(max(blk, 0), max_block);  // never address outside the pool
     const int64_t slot =
-        PAGED ? ((int64_t(blk) << bs_log2) | (key & ((1 << bs_log2) - 1))) : int64_t(key);
+        PAGED ? ((int64_t(b) << bs_log2) | (key & ((1 << bs_log2) - 1))) : int64_t(key);
     const size_t off = size_t(slot) * row_bytes + 32 * (tid & 3);
     t.k0 = *reinterpret_cast<const uint4*>(kb + off);
     t.k1 = *reinterpret_cast<const uint4*>(kb + off + 16);
@@ -554,22 +555,23 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_attention_kernel(const 
     Fp8Tile f8;
     const int key_lo = kt_lo * kPfKeys;
     if constexpr (FP8) {
-        if constexpr (PAGED) blk8 = table_block(a, min(key_lo + (tid >> 2), a.kv_len - 1));
-        fp8_load<PAGED>(kb, vb, a.kv_row_bytes, key_lo, a.kv_len, tid, blk8, a.bs_log2, f8);
+        if constexpr (PAGED) blk8 = table_entry(a, min(key_lo + (tid >> 2), a.kv_len - 1));
+        fp8_load<PAGED>(kb, vb, a.kv_row_bytes, key_lo, a.kv_len, tid, blk8, a.bs_log2,
+                        a.max_block, f8);
         fp8_store(s_lds, s_lds + kVBase, tid, f8);
         if constexpr (PAGED)
             if (kt_lo + 1 < n_kt)
-                blk8 = table_block(a, min(key_lo + kPfKeys + (tid >> 2), a.kv_len - 1));
+                blk8 = table_entry(a, min(key_lo + kPfKeys + (tid >> 2), a.kv_len - 1));
     } else {
         if constexpr (PAGED)
-            tile_blocks(a.table, a.bs_log2, a.max_block, kt_lo, a.kv_len, wave, lane, blk);
+            tile_blocks(a.table, a.bs_log2, kt_lo, a.kv_len, wave, lane, blk);
         dma_tile<true, PAGED>(kb, a.kv_row_bytes, key_lo, a.kv_len, wave, lane, s_lds, blk,
-                              a.bs_log2);
+                              a.bs_log2, a.max_block);
         dma_tile<false, PAGED>(vb, a.kv_row_bytes, key_lo, a.kv_len, wave, lane, s_lds + kVBase,
-                               blk, a.bs_log2);
+                               blk, a.bs_log2, a.max_block);
         if constexpr (PAGED)
             if (kt_lo + 1 < n_kt)
-                tile_blocks(a.table, a.bs_log2, a.max_block, kt_lo + 1, a.kv_len, wave, lane, blk);
+                tile_blocks(a.table, a.bs_log2, kt_lo + 1, a.kv_len, wave, lane, blk);
     }
     if (a.cos_t) {  // packed partials with RoPE (wave-uniform)
         // Whole 32-bit words in and out: two fp16 elements per word, low half
@@ -635,24 +637,25 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_attention_kernel(const 
         constexpr int BUF = decltype(buf_c)::value;
         // This wave's tile loads have landed in LDS; the barrier covers the others'
         // and frees the other buffer (read in the previous step) for the next tile.
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_dma_wait();
         __syncthreads();
         if (kt + 1 < n_kt) {
             if constexpr (FP8) {
                 fp8_load<PAGED>(kb, vb, a.kv_row_bytes, (kt + 1) * kPfKeys, a.kv_len, tid, blk8,
-                                a.bs_log2, f8);
+                                a.bs_log2, a.max_block, f8);
                 if constexpr (PAGED)
                     if (kt + 2 < n_kt)
-                        blk8 = table_block(a, min((kt + 2) * kPfKeys + (tid >> 2), a.kv_len - 1));
+                        blk8 = table_entry(a, min((kt + 2) * kPfKeys + (tid >> 2), a.kv_len - 1));
             } else {
                 dma_tile<true, PAGED>(kb, a.kv_row_bytes, (kt + 1) * kPfKeys, a.kv_len, wave, lane,
-                                      s_lds + (BUF ^ 1) * kTileBytes, blk, a.bs_log2);
+                                      s_lds + (BUF ^ 1) * kTileBytes, blk, a.bs_log2,
+                                      a.max_block);
                 dma_tile<false, PAGED>(vb, a.kv_row_bytes, (kt + 1) * kPfKeys, a.kv_len, wave,
                                        lane, s_lds + kVBase + (BUF ^ 1) * kTileBytes, blk,
-                                       a.bs_log2);
+                                       a.bs_log2, a.max_block);
                 if constexpr (PAGED)
                     if (kt + 2 < n_kt)
-                        tile_blocks(a.table, a.bs_log2, a.max_block, kt + 2, a.kv_len, wave, lane,
+                        tile_blocks(a.table, a.bs_log2, kt + 2, a.kv_len, wave, lane,
                                     blk);
             }
         }
