@@ -86,13 +86,17 @@ __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32
                  : "memory");
 }
 
-// Waits for the wave's vector-memory operations, the DMA above among them (the
-// builtin, so that the compiler also knows its own loads have arrived).
-__device__ __forceinline__ void lds_dma_wait() {
+// Waits until at most N of the wave's vector-memory operations are outstanding
+// (they retire in issue order), the DMA above among them. The builtin, so that
+// the compiler also knows which of its own loads have arrived.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N >= 0 && N < 64, "vmcnt has six bits");
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), other counters free
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));  // other counters free
     asm volatile("" ::: "memory");
 }
+__device__ __forceinline__ void lds_dma_wait() { wait_vmcnt<0>(); }
 
 // ---- cross-lane reductions (wave64) -----------------------------------------
 // DPP move of v (row_mask, bank_mask all lanes; bound_ctrl: a source lane

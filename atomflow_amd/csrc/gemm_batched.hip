@@ -11,7 +11,9 @@
 // and writes K and V to each token's slot of the paged pool, exactly as
 // af_paged_rope_append does on the projection's output.
 //
-// Design (HBM-bound: one weight byte per 2*M flops; M <= 32 per launch tile):
+// Few tokens (w8a16_batched_kernel; HBM-bound: one weight byte per 2*M flops, M
+// <= 32 per workgroup). Launches of more tokens or rows take the tiled kernel
+// further down (pick_tile):
 //  * D = X W^T on v_mfma_f32_16x16x32_f16: A = 16 tokens x 32 k of x (read
 //    from L2; rows past m repeat row m-1 and are not stored), B = 32 k x 16
 //    weight rows (E4M3 -> fp16 in registers with v_cvt_scalef32_pk_f16_fp8 at
@@ -42,6 +44,7 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v_t __attribute__((ext_vector_type(2)));
 
 typedef float float4v_t __attribute__((ext_vector_type(4)));
+typedef float float16v_t __attribute__((ext_vector_type(16)));
 
 constexpr int kBgParts = 8;               // K parts = waves per workgroup
 constexpr int kBgThreads = 64 * kBgParts;  // 512
@@ -70,6 +73,9 @@ struct BatchedArgs {
     const float* k_scales;  // fp8 pools: [n_kv_heads]
     const float* v_scales;
     int32_t* d_status;
+    // Tiled kernel: y (and in the fused kernel the tables and the pool) allow
+    // 16-byte accesses.
+    int32_t vec;
 };
 
 // Eight E4M3 codes (two dwords) -> eight fp16 values, exact.
@@ -315,8 +321,503 @@ __global__ __launch_bounds__(kBgThreads, 4) void w8a16_batched_kernel(const Batc
     }
 }
 
+// ---- many tokens: a tiled contraction ------------------------------------------
+//
+// From a few dozen tokens on the projection is no longer the weight stream with a
+// little arithmetic: each workgroup re-reads the activations of its tokens (the
+// 16-row kernel above reads all of x per 16 rows and the weights once per 32
+// tokens), and the matrix cores have work. The tiled kernel gives a workgroup BM
+// tokens x BN weight rows and, with KS > 1, KS group-aligned parts of K; a wave
+// owns a (BM / WR) x (BN / WC) piece of one part as 32x32x16 MFMAs. 2011 tokens
+// of 8192 x 3072: 470 us on the 16-row kernel, 108 here (0.95 PFLOP/s); a bare
+// loop of the same MFMAs and barriers takes 77, the DMA, the operand reads and
+// the group scales about 10 each; 64 tokens of 3072 x 8192: 25.7 and 16.6 us.
+//  * K advances 64 per step. A step's x rows (128 B each, fp16) and weight rows
+//    (64 B each, E4M3) go from global memory straight into LDS (lds_dma16), in a
+//    ring of ST stages: the loads of step s + ST - 1 are issued in step s, one
+//    barrier per step. The weights stay E4M3 in LDS (half the LDS traffic of
+//    fp16) and convert in registers, exactly.
+//  * 16-byte chunks are XOR-swizzled (x by row / 2, weights by row / 4) so that
+//    an operand read of 16 rows covers every bank once; the swizzle is made by
+//    choosing which chunk each DMA lane fetches.
+//  * A lane reads 16 weight bytes for two MFMAs: of 32 k, lanes 0-31 hold the
+//    first 16 and lanes 32-63 the last; x is read in the same k order.
+//  * Group scales: D's column is the lane's weight row, so a group's scale is
+//    one value per lane and column tile. The accumulator is kept in units of
+//    the current group's scale: entering group g it is multiplied by
+//    scale[g-1] / scale[g] (one multiply per element and group), at the end by
+//    the last scale. (A second accumulator per group, added with its scale,
+//    would double the accumulator registers.) A zero scale counts as 2^-66,
+//    whose group then adds less than half the smallest fp16. Scales are staged
+//    in LDS eight groups at a time: a register load waited for in each group
+//    would drain the DMA ring with it.
+//  * The parts of K are summed through LDS in a fixed order, and the tile leaves
+//    through LDS as fp16, so rows are stored 16 B per lane. In the fused kernel
+//    the BN columns are BN / 2 dims d of a head and their partners d + 64, and
+//    each thread rotates and appends 8 such pairs of a token from there.
+//  * Workgroups are dealt so that each XCD owns whole column panels (its L2
+//    then reads each weight once and x once).
+constexpr float kZeroScale = 0x1p-66f;
+constexpr int kScaleChunk = 8;  // groups staged at a time
+
+template <int BM, int BN, int KS, int ST>
+struct TileLayout {
+    static constexpr int kXBytes = BM * 128;  // one step of x rows
+    static constexpr int kWBytes = BN * 64;   // one step of weight rows
+    static constexpr int kPart = kXBytes + kWBytes;
+    static constexpr int kStage = KS * kPart;
+    static constexpr int kRing = ST * kStage;
+    static constexpr int kOutStride = BN * 2 + 16;  // bytes between output rows in LDS
+    static constexpr int kRed = KS > 1 ? KS * BM * BN * 4 : 0;
+    static constexpr int kTail = kRed + BM * kOutStride;
+    static constexpr int kScales = kRing;  // [2][KS][kScaleChunk][BN] fp16 after the ring
+    static constexpr int kScaleBytes = ST > 2 ? 2 * KS * kScaleChunk * BN * 2 : 0;
+    static constexpr int kLds =
+        kRing + kScaleBytes > kTail ? kRing + kScaleBytes : kTail;
+};
+
+// The weight row of column c of panel pn: the fused kernel's panels hold dims
+// sub * BN / 2 .. of one head (columns below BN / 2) and their rotation partners.
+template <bool FUSED, int BN>
+__device__ __forceinline__ int panel_row(int pn, int c) {
+    if constexpr (!FUSED) return pn * BN + c;
+    constexpr int H = BN / 2, SUBS = 64 / H;
+    return (pn / SUBS) * 128 + (pn % SUBS) * H + (c % H) + (c / H) * 64;
+}
+
+// Stores the tile's fp16 rows from LDS.
+template <int BM, int BN, int THREADS, int STRIDE>
+__device__ __forceinline__ void store_tile(const BatchedArgs& a, const char* s_out, int t0, int n0,
+                                           int tid) {
+    constexpr int kChunks = BN / 8;
+    for (int c = tid; c < BM * kChunks; c += THREADS) {
+        const int r = c / kChunks, q = c % kChunks;
+        const int t = t0 + r, col = n0 + 8 * q;
+        if (t >= a.m || col >= a.n) continue;
+        const uint4 v = *reinterpret_cast<const uint4*>(s_out + r * STRIDE + 16 * q);
+        uint16_t* dst = a.y + size_t(t) * a.y_stride + col;
+        if (a.vec && col + 8 <= a.n) {
+            *reinterpret_cast<uint4*>(dst) = v;
+        } else {
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (col + e < a.n) dst[e] = uint16_t(w[e >> 1] >> (16 * (e & 1)));
+        }
+    }
+}
+
+// Rotates the tile's Q and K pairs from LDS, stores them, appends K and V.
+template <bool FP8, int BM, int BN, int THREADS, int STRIDE>
+__device__ __forceinline__ void store_tile_rope(const BatchedArgs& a, const char* s_out, int t0,
+                                                int pn, int tid) {
+    constexpr int H = BN / 2, SUBS = 64 / H, kChunks = H / 8;
+    const int head = pn / SUBS;
+    const int kind = head < a.n_q_heads ? 0 : (head < a.n_q_heads + a.n_kv_heads ? 1 : 2);
+    const int kh = head - a.n_q_heads - (kind == 2 ? a.n_kv_heads : 0);
+    const int kv_dim = a.n_kv_heads * 128;
+    for (int c = tid; c < BM * kChunks; c += THREADS) {
+        const int r = c / kChunks, q = c % kChunks;
+        const int d = (pn % SUBS) * H + 8 * q;  // pairs (d .. d + 7, d + 64 ..)
+        const int t = t0 + r;
+        if (t >= a.m) continue;
+        const char* row = s_out + r * STRIDE + 16 * q;
+        const uint4 vx = *reinterpret_cast<const uint4*>(row);
+        const uint4 vy = *reinterpret_cast<const uint4*>(row + 2 * H);
+        const uint32_t xw[4] = {vx.x, vx.y, vx.z, vx.w}, yw[4] = {vy.x, vy.y, vy.z, vy.w};
+        uint32_t xo[4] = {vx.x, vx.y, vx.z, vx.w}, yo[4] = {vy.x, vy.y, vy.z, vy.w};
+        const int pos = a.d_positions[t];
+        const int64_t slot = a.d_slots[t];
+        // nothing is rotated or appended for an out-of-range token
+        const bool ok = pos >= 0 && pos < a.max_pos && slot >= 0 && slot < a.max_rows;
+        if (!ok && a.d_status) *a.d_status = AF_ERR_OUT_OF_RANGE;
+        if (ok && kind < 2) {
+            const float* cr = a.cos_t + size_t(pos) * 64 + d;
+            const float* sr = a.sin_t + size_t(pos) * 64 + d;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                uint16_t x0, y0, x1, y1;
+                rope_rotate(uint16_t(xw[w]), uint16_t(yw[w]), cr[2 * w], sr[2 * w], x0, y0);
+                rope_rotate(uint16_t(xw[w] >> 16), uint16_t(yw[w] >> 16), cr[2 * w + 1],
+                            sr[2 * w + 1], x1, y1);
+                xo[w] = uint32_t(x0) | (uint32_t(x1) << 16);
+                yo[w] = uint32_t(y0) | (uint32_t(y1) << 16);
+            }
+        }
+        auto put = [&](uint16_t* dst, const uint32_t (&v)[4]) {
+            if (a.vec) {
+                *reinterpret_cast<uint4*>(dst) = make_uint4(v[0], v[1], v[2], v[3]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) dst[e] = uint16_t(v[e >> 1] >> (16 * (e & 1)));
+            }
+        };
+        uint16_t* yrow = a.y + size_t(t) * a.y_stride + head * 128 + d;
+        put(yrow, xo);
+        put(yrow + 64, yo);
+        if (!ok || kind == 0) continue;
+        const size_t e0 = size_t(slot) * kv_dim + size_t(kh) * 128 + d;
+        uint8_t* base = kind == 1 ? a.k_dst : a.v_dst;
+        if constexpr (FP8) {
+            const float sc = (kind == 1 ? a.k_scales : a.v_scales)[kh];
+            auto put8 = [&](uint8_t* dst, const uint32_t (&v)[4]) {
+                uint32_t code[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    code[e] = quantize_fp8(uint16_t(v[e >> 1] >> (16 * (e & 1))), sc);
+                if (a.vec) {
+                    *reinterpret_cast<uint2*>(dst) =
+                        make_uint2(code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24),
+                                   code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) dst[e] = uint8_t(code[e]);
+                }
+            };
+            put8(base + e0, xo);
+            put8(base + e0 + 64, yo);
+        } else {
+            put(reinterpret_cast<uint16_t*>(base) + e0, xo);
+            put(reinterpret_cast<uint16_t*>(base) + e0 + 64, yo);
+        }
+    }
+}
+
+// WGS: workgroups per CU the registers are budgeted for.
+template <bool FUSED, bool FP8, int BM, int BN, int WR, int WC, int KS, int ST, int WGS>
+__global__ __launch_bounds__(64 * WR * WC * KS, (WGS * WR * WC * KS + 3) / 4) void
+w8a16_tiled_kernel(const BatchedArgs a) {
+    using L = TileLayout<BM, BN, KS, ST>;
+    constexpr int NW = WR * WC, THREADS = 64 * NW * KS;
+    constexpr int MT = BM / WR / 32, NT = BN / WC / 32;  // 32x32 tiles of a wave
+    constexpr int XI = BM / 8 / NW, WI = BN / 16 / NW;   // DMA instructions of a wave per step
+    constexpr int D = ST - 1;           // steps in flight ahead
+    // With one step in flight every step waits for all of its wave's loads, so a
+    // register load of the next group's scales costs no wait of its own.
+    constexpr bool kRegScales = ST == 2;
+    static_assert(ST >= 2, "a stage is read while the next one loads");
+    static_assert(MT >= 1 && NT >= 1 && XI >= 1 && WI >= 1, "tile too small for its waves");
+    static_assert(XI * 8 * NW == BM && WI * 16 * NW == BN && BN <= 64 * NW, "uneven DMA");
+    __shared__ __align__(16) char s_lds[L::kLds];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = KS > 1 ? wid / NW : 0, wave = KS > 1 ? wid % NW : wid;
+    const int col = lane & 31, hi = lane >> 5;
+    // Tile of this workgroup: workgroup ids go round-robin over the 8 XCDs, so
+    // the ids of one XCD take one contiguous range of tiles, token tiles fastest.
+    const int mb = (a.m + BM - 1) / BM;
+    const int tiles = mb * ((a.n + BN - 1) / BN);
+    const int xcd = int(blockIdx.x) & 7, per = tiles >> 3, rest = tiles & 7;
+    const int tile = xcd * per + min(xcd, rest) + (int(blockIdx.x) >> 3);
+    const int t0 = (tile % mb) * BM, pn = tile / mb;
+
+    // This wave's part of K, in groups and 64-k steps.
+    const int g_lo = ks * a.groups / KS, g_hi = (ks + 1) * a.groups / KS;
+    const int per_group = a.group_size / 64;
+    const int steps = (g_hi - g_lo) * per_group;
+    const int all_steps = (a.groups + KS - 1) / KS * per_group;  // the longest part's
+
+    // DMA sources: one scalar base per operand, 32-bit lane offsets. Rows past m
+    // or n load the last row: their products are not stored.
+    const char* xb = reinterpret_cast<const char*>(a.x + size_t(t0) * a.x_stride) +
+                     size_t(g_lo) * a.group_size * 2;
+    const int n_first = panel_row<FUSED, BN>(pn, 0);
+    const char* wb = reinterpret_cast<const char*>(a.w + size_t(n_first) * a.k) +
+                     size_t(g_lo) * a.group_size;
+    uint32_t xoff[XI], woff[WI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int r = 8 * (wave * XI + i) + (lane >> 3);
+        const int chunk = (lane & 7) ^ ((r >> 1) & 7);
+        xoff[i] = uint32_t(min(r, a.m - 1 - t0)) * uint32_t(a.x_stride) * 2u + 16u * chunk;
+    }
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+        const int r = 16 * (wave * WI + i) + (lane >> 2);
+        const int chunk = (lane & 3) ^ ((r >> 2) & 3);
+        woff[i] = uint32_t(min(panel_row<FUSED, BN>(pn, r), a.n - 1) - n_first) * uint32_t(a.k) +
+                  16u * chunk;
+    }
+    const uint32_t lds0 = lds_address(s_lds) + ks * L::kPart;
+    auto issue = [&](int step, int buf) {
+        const uint32_t dst = lds0 + buf * L::kStage;
+        const char* xs = xb + size_t(step) * 128;
+        const char* ws = wb + size_t(step) * 64;
+#pragma unroll
+        for (int i = 0; i < XI; ++i) lds_dma16(xs, xoff[i], dst + 1024 * (wave * XI + i));
+#pragma unroll
+        for (int i = 0; i < WI; ++i)
+            lds_dma16(ws, woff[i], dst + L::kXBytes + 1024 * (wave * WI + i));
+    };
+
+    // Scales of chunk c (groups g_lo + 8 c ..) of this thread's weight row.
+    const int lt = tid - ks * 64 * NW;  // thread within the part
+    const bool has_row = lt < BN;
+    const uint16_t* srow =
+        a.scales + size_t(min(panel_row<FUSED, BN>(pn, min(lt, BN - 1)), a.n - 1)) * a.groups;
+    uint16_t* s_scale = reinterpret_cast<uint16_t*>(s_lds + L::kScales);
+    uint16_t next_sc[kScaleChunk];
+    auto load_scales = [&](int c) {
+        if (has_row)
+#pragma unroll
+            for (int i = 0; i < kScaleChunk; ++i)
+                next_sc[i] = srow[min(g_lo + c * kScaleChunk + i, a.groups - 1)];
+    };
+    auto stage_scales = [&](int c) {
+        if (has_row)
+#pragma unroll
+            for (int i = 0; i < kScaleChunk; ++i)
+                s_scale[(((c & 1) * KS + ks) * kScaleChunk + i) * BN + lt] = next_sc[i];
+    };
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+        if (i < steps) issue(i, i);
+    if constexpr (!kRegScales) {
+        load_scales(0);
+        stage_scales(0);
+        load_scales(1);
+    }
+
+    // Operand reads: x row wm + 32 mt + col, weight row wn + 32 nt + col.
+    const int wm = (wave / WC) * (BM / WR), wn = (wave % WC) * (BN / WC);
+    const int xr = wm + col, wr = wn + col;  // (32 mt does not change (row / 2) % 8)
+    uint32_t xa[4], wa[2];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // q = 2 p + j: 16-byte chunk 4 p + 2 hi + j
+        const int chunk = 4 * (q >> 1) + 2 * hi + (q & 1);
+        xa[q] = ks * L::kPart + uint32_t(xr) * 128u + 16u * uint32_t(chunk ^ ((xr >> 1) & 7));
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+        wa[p] = ks * L::kPart + L::kXBytes + uint32_t(wr) * 64u +
+                16u * uint32_t((2 * p + hi) ^ ((wr >> 2) & 3));
+
+    float16v_t acc[MT][NT];
+    float scale[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        scale[nt] = 1.0f;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
+    }
+
+    uint16_t sraw[NT];  // kRegScales: the next group's scales
+    const uint16_t* slane[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        slane[nt] = a.scales +
+                    size_t(min(panel_row<FUSED, BN>(pn, wr + 32 * nt), a.n - 1)) * a.groups;
+        if constexpr (kRegScales) sraw[nt] = slane[nt][min(g_lo, a.groups - 1)];
+    }
+    int left = 0;    // steps of the current group still to come
+    int group = -1;  // the current group of the part
+    int buf = 0;
+    for (int st = 0; st < all_steps; ++st) {
+        // This step's loads have arrived (the D - 1 later steps' may be in
+        // flight); the barrier covers the other waves' and frees the buffer read
+        // a step ago.
+        if (st + D - 1 < steps) wait_vmcnt<(D - 1) * (XI + WI)>();
+        else wait_vmcnt<0>();
+        __syncthreads();
+        if (KS > 1 && st >= steps) continue;  // a shorter part waits for the others
+        if (left == 0) {  // a group begins: the accumulator moves to its scale
+            left = per_group;
+            ++group;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                float v;
+                if constexpr (kRegScales)
+                    v = h2f(sraw[nt]);
+                else
+                    v = h2f(s_scale[((((group / kScaleChunk) & 1) * KS + ks) * kScaleChunk +
+                                     group % kScaleChunk) * BN + wr + 32 * nt]);
+                const float sc = v == 0.0f ? kZeroScale : v;
+                if (group > 0) {
+                    const float ratio = scale[nt] / sc;
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) acc[mt][nt][r] *= ratio;
+                }
+                scale[nt] = sc;
+                if constexpr (kRegScales)
+                    sraw[nt] = slane[nt][min(g_lo + group + 1, a.groups - 1)];
+            }
+            if constexpr (!kRegScales)
+                if (group % kScaleChunk == kScaleChunk - 1) {  // read a group later
+                    const int c = group / kScaleChunk + 1;
+                    stage_scales(c);
+                    load_scales(c + 1);
+                }
+        }
+        --left;
+        if (st + D < steps) issue(st + D, buf == 0 ? D : buf - 1);
+        const char* s = s_lds + buf * L::kStage;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            half8_t wf[NT][2];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const uint4 v = *reinterpret_cast<const uint4*>(s + wa[p] + nt * 32 * 64);
+                wf[nt][0] = e4m3x8(v.x, v.y);
+                wf[nt][1] = e4m3x8(v.z, v.w);
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const half8_t xf = __builtin_bit_cast(
+                        half8_t,
+                        *reinterpret_cast<const uint4*>(s + xa[2 * p + j] + mt * 32 * 128));
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf, wf[nt][j],
+                                                                             acc[mt][nt], 0, 0, 0);
+                }
+        }
+        buf = buf == D ? 0 : buf + 1;
+    }
+
+    // Register r of (mt, nt) is token 32 mt + 8 (r / 4) + 4 hi + r % 4 of the
+    // wave's piece, column 32 nt + col.
+    __syncthreads();
+    char* s_out = s_lds + L::kRed;
+    auto put = [&](int mt, int nt, int r, float v) {
+        const int row = wm + 32 * mt + 8 * (r >> 2) + 4 * hi + (r & 3);
+        *reinterpret_cast<uint16_t*>(s_out + row * L::kOutStride + 2 * (wr + 32 * nt)) = f2h(v);
+    };
+    if constexpr (KS == 1) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) put(mt, nt, r, acc[mt][nt][r] * scale[nt]);
+    } else {
+        // Every part leaves its sums in LDS; each part's waves add a 16 / KS
+        // share of the registers over the parts, part 0 first.
+        float* red = reinterpret_cast<float*>(s_lds);
+        auto at = [&](int part, int mt, int nt, int r) {
+            return ((((part * NW + wave) * MT + mt) * NT + nt) * 16 + r) * 64 + lane;
+        };
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) red[at(ks, mt, nt, r)] = acc[mt][nt][r] * scale[nt];
+        __syncthreads();
+        constexpr int RS = 16 / KS;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int i = 0; i < RS; ++i) {
+                    const int r = ks * RS + i;
+                    float v = red[at(0, mt, nt, r)];
+#pragma unroll
+                    for (int part = 1; part < KS; ++part) v += red[at(part, mt, nt, r)];
+                    put(mt, nt, r, v);
+                }
+    }
+    __syncthreads();
+    if constexpr (FUSED)
+        store_tile_rope<FP8, BM, BN, THREADS, L::kOutStride>(a, s_out, t0, pn, tid);
+    else
+        store_tile<BM, BN, THREADS, L::kOutStride>(a, s_out, t0, pn * BN, tid);
+}
+
+template <bool FUSED, bool FP8, int BM, int BN, int WR, int WC, int KS, int ST, int WGS>
+void launch_tiled(const BatchedArgs& a, hipStream_t s) {
+    const int tiles = ((a.m + BM - 1) / BM) * ((a.n + BN - 1) / BN);
+    hipLaunchKernelGGL((w8a16_tiled_kernel<FUSED, FP8, BM, BN, WR, WC, KS, ST, WGS>), dim3(tiles),
+                       dim3(64 * WR * WC * KS), 0, s, a);
+}
+
+// The tiles, and what a launch of each was measured to cost on MI355X (nine
+// (n, k) shapes from 2048 x 8192 to 14336 x 4096, 16 to 4000 tokens; the model
+// below fits each within 5-9 % rms): a round of workgroups, `wgs` of them per CU
+// while tiles last, takes `round` plus per 64-k step `step` and, for each
+// workgroup that shares the CU, `share` (us); a launch `fixed` besides. Small
+// tiles with several parts of K fill the device when tokens or rows are few
+// (their weights and x are then read by more workgroups), large ones read the
+// least and keep the matrix cores busiest.
+struct TileCost {
+    int bm, bn, ks, wgs;
+    float fixed, step, share, round;
+};
+enum { kT128x256, kT128x128, kT64x128, kT64x64k2, kT128x64k2, kT64x64k4, kT64x32k4, kT32x32k4,
+       kT32x32k8, kTiles };
+constexpr TileCost kTileCost[kTiles] = {
+    {128, 256, 1, 2, 0.0f, 0.0f, 0.940f, 5.94f},      {128, 128, 1, 3, 0.0f, 0.234f, 0.447f, 3.20f},
+    {64, 128, 1, 4, 0.0f, 0.346f, 0.185f, 1.57f},     {64, 64, 2, 2, 0.83f, 0.180f, 0.312f, 2.65f},
+    {128, 64, 2, 1, 0.0f, 0.698f, 0.0f, 4.33f},       {64, 64, 4, 1, 0.0f, 0.923f, 0.0f, 3.13f},
+    {64, 32, 4, 1, 0.71f, 0.582f, 0.0f, 2.59f},       {32, 32, 4, 2, 2.11f, 0.161f, 0.282f, 1.30f},
+    {32, 32, 8, 1, 1.41f, 0.759f, 0.0f, 2.60f}};
+
+// The cheapest tile by kTileCost, or -1 for the 16-row kernel above: group sizes
+// that are not whole 64-k steps, strides past the 32-bit lane offsets, and
+// launches of at most one 16-row workgroup per CU, whose eight K parts then
+// stream the weights faster than any tile (3072 rows of k 3072: 16 tokens 6.1 us
+// against 7.0, 32 tokens 7.0 against 7.8; at 48 tokens, past one workgroup per
+// CU, 10.3 against 7.9). The choice depends on (m, n, k, group size) alone, so
+// the fused kernel and the plain projection always sum in the same order.
+int pick_tile(const BatchedArgs& a) {
+    if (a.group_size % 64 != 0 || a.x_stride >= (int64_t(1) << 23) || a.k >= (1 << 24) ||
+        int64_t(a.m) * a.n >= (int64_t(1) << 40))
+        return -1;
+    const unsigned cus = unsigned(device_compute_units());
+    if (int64_t(ceil_div(a.n, kBgRows)) * ceil_div(a.m, 2 * kBgTile) <= int64_t(cus)) return -1;
+    // (called for every launch: constant tile sizes, 32-bit arithmetic)
+    const unsigned m = unsigned(a.m), n = unsigned(a.n), groups = unsigned(a.groups);
+    const float per_group = float(a.group_size / 64);
+    int best = 0;
+    float best_cost = 0.0f;
+#pragma clang loop unroll(full)
+    for (int i = 0; i < kTiles; ++i) {
+        constexpr auto up = [](unsigned x, int by) { return (x + by - 1) / unsigned(by); };
+        const TileCost& c = kTileCost[i];
+        const unsigned tiles = up(m, c.bm) * up(n, c.bn);  // (m n < 2^40 over 32 x 32 at least)
+        const unsigned per_cu = (tiles + cus - 1) / cus;   // shares of the launch's busiest CUs
+        const unsigned rounds = up(per_cu, c.wgs);
+        const float steps = float(up(groups, c.ks)) * per_group;
+        const float cost = c.fixed + float(rounds) * (c.round + steps * c.step) +
+                           float(per_cu) * steps * c.share;
+        if (i == 0 || cost < best_cost) {
+            best = i;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+template <bool FUSED, bool FP8>
+void launch_tile(int tile, const BatchedArgs& a, hipStream_t s) {
+    switch (tile) {
+        case kT128x256:
+            // (a fused panel is at most one head; the same sums in 128 columns)
+            if constexpr (!FUSED) return launch_tiled<FUSED, FP8, 128, 256, 2, 4, 1, 2, 2>(a, s);
+            [[fallthrough]];
+        case kT128x128: return launch_tiled<FUSED, FP8, 128, 128, 1, 4, 1, 2, 3>(a, s);
+        case kT64x128: return launch_tiled<FUSED, FP8, 64, 128, 1, 4, 1, 2, 4>(a, s);
+        case kT64x64k2: return launch_tiled<FUSED, FP8, 64, 64, 2, 2, 2, 3, 2>(a, s);
+        case kT128x64k2: return launch_tiled<FUSED, FP8, 128, 64, 2, 2, 2, 3, 1>(a, s);
+        case kT64x64k4: return launch_tiled<FUSED, FP8, 64, 64, 2, 1, 4, 3, 1>(a, s);
+        case kT64x32k4: return launch_tiled<FUSED, FP8, 64, 32, 2, 1, 4, 3, 1>(a, s);
+        case kT32x32k4: return launch_tiled<FUSED, FP8, 32, 32, 1, 1, 4, 3, 2>(a, s);
+        default: return launch_tiled<FUSED, FP8, 32, 32, 1, 1, 8, 3, 1>(a, s);
+    }
+}
+
 template <bool FUSED, bool FP8>
 void launch_batched(const BatchedArgs& a, int row_blocks, hipStream_t s) {
+    const int tile = pick_tile(a);
+    if (tile >= 0) return launch_tile<FUSED, FP8>(tile, a, s);
     const bool two = a.m > kBgTile;
     const int per = kBgTile * (two ? 2 : 1);
     const dim3 grid(row_blocks, (a.m + per - 1) / per), block(kBgThreads);
@@ -373,6 +874,7 @@ extern "C" int af_w8a16_gemm_batched(const void* x, int64_t x_stride, int m, con
     fill_common(a, x, x_stride, m, weight, scales, n, k, group_size);
     a.y = static_cast<uint16_t*>(y);
     a.y_stride = y_stride;
+    a.vec = aligned16(y) && y_stride % 8 == 0;
     launch_batched<false, false>(a, (n + kBgRows - 1) / kBgRows, static_cast<hipStream_t>(stream));
     AF_TRY_LAUNCH();
     return AF_OK;
@@ -451,6 +953,8 @@ extern "C" int af_paged_qkv_rope_append(const void* x, int64_t x_stride, int m,
         a.v_scales = a.k_scales + pool->n_kv_heads;
     }
     a.d_status = d_status;
+    a.vec = aligned16(qkv_out) && aligned16(cos_table) && aligned16(sin_table) &&
+            aligned16(pool->base);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (fp8)
         launch_batched<true, true>(a, n / kBgRows, s);  // eight workgroups per head

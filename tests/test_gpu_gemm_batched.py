@@ -193,3 +193,84 @@ def test_paged_qkv_rope_append_graph_replays(gpu):
         assert np.array_equal(bufs[0].download(np.uint8, (pool_bytes,)),
                               bufs[1].download(np.uint8, (pool_bytes,))), f"replay {step}"
     graph.destroy()
+
+
+def deq(w, s, group):
+    """float64 weights of E4M3 codes and fp16 group scales."""
+    n, k = w.shape
+    table = oracle.e4m3_decode_table().astype(np.float64)
+    return (table[w].reshape(n, k // group, group) * s.astype(np.float64)[:, :, None]).reshape(n, k)
+
+
+@pytest.mark.parametrize("n,k,m,group,y_off", [
+    (4100, 64, 2, 64, 0), (4100, 640, 33, 128, 1), (4100, 640, 2, 128, 0), (1000, 640, 520, 128, 1),
+    (1000, 1024, 520, 128, 0), (4100, 3072, 2, 128, 0), (8200, 1536, 65, 512, 0),
+    (8200, 3072, 65, 128, 0), (4100, 128, 2100, 128, 0), (3072, 3072, 2100, 128, 0)])
+def test_gemm_tiled_parity(gpu, n, k, m, group, y_off):
+    """One case or more for each tile of the tiled kernel, with partial token and
+    column tiles, fewer groups than K parts, parts of unequal length, output rows
+    that are not 16-byte aligned, and a zero and a very small group scale. Every
+    output within half an fp16 ulp plus the fp32 summation bound; bytes around the
+    outputs are untouched."""
+    say(f"tiled gemm n={n} k={k} m={m} group={group} y offset {y_off}")
+    w, _, s = gemv_case(n, k, 0xA70F40 + n + k, group=group)
+    s = s.copy()
+    s[1, 0] = 0.0
+    s[2, -1] = np.float16(6e-8)
+    x = np.random.default_rng(m + n).standard_normal((m, k)).astype(np.float16)
+    stride = n + (5 if y_off else 8)
+    y = dev.DeviceBuffer((m * stride + y_off + 1) // 2 * 4)
+    y.fill_u32(0x7a7a7a7a)
+    kv.launch_w8a16_gemm_batched(up(x), k, m, up(w), up(s), y.ptr + 2 * y_off, stride, n, k, group)
+    raw = y.download(np.uint16)
+    assert np.all(raw[:y_off] == 0x7a7a)
+    rows = np.lib.stride_tricks.as_strided(raw[y_off:], (m, n), (2 * stride, 2)).copy()
+    pad = np.lib.stride_tricks.as_strided(raw[y_off + n:], (m, stride - n), (2 * stride, 2))
+    assert np.all(pad == 0x7a7a)
+    got = rows.view(np.float16).astype(np.float64)
+    assert np.all(np.isfinite(got))
+    wd = deq(w, s, group)
+    want = x.astype(np.float64) @ wd.T
+    bound = k * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(wd).T)
+    err = np.abs(got - want)
+    assert np.all(err <= 0.5 * fp16_ulp(want) + bound), f"max err {err.max():.3e}"
+
+
+@pytest.mark.parametrize("fp8,m,q_off", [(False, 17, 0), (True, 40, 0), (True, 65, 0), (False, 131, 1),
+                                         (True, 300, 1), (False, 513, 0), (True, 1100, 0)])
+def test_paged_qkv_rope_append_many_tokens(gpu, fp8, m, q_off):
+    """The tiled fused form: bit for bit the batched projection followed by the
+    paged append, whole pool compared, with tokens out of range at both ends;
+    q_off: qkv rows that are not 16-byte aligned."""
+    k_in, bs, total, max_pos = 3072, 16, 96, 700
+    say(f"paged qkv rope append of {m} tokens, fp8 {fp8}")
+    w, _, s = gemv_case(QKV, k_in, 0xA70F33, group=128)
+    xs = np.random.default_rng(13).standard_normal((m, k_in)).astype(np.float16)
+    r = np.random.default_rng(14)
+    slots = r.permutation(total * bs)[:m].astype(np.int64)
+    positions = r.integers(0, max_pos, m).astype(np.int32)
+    positions[7], slots[m - 1] = max_pos, total * bs
+    pool_bytes = 2 * 2 * total * bs * KV_DIM * (1 if fp8 else 2)
+    init = r.integers(0, 256, pool_bytes, dtype=np.uint8)
+    scales = up(np.full((2, 2, NKV), 0.04, np.float32)) if fp8 else None
+    dtype = atomflow_amd.AF_KV_FP8_E4M3 if fp8 else atomflow_amd.AF_KV_FP16
+    pools = []
+    for _ in range(2):
+        buf = up(init)
+        pools.append((buf, kv.make_pool(buf, dtype, bs, 2, NKV, HD, total, scales)))
+    c, sn = oracle.rope_table(max_pos, HD, THETA)
+    d_c, d_s, dx, dw, ds = up(c), up(sn), up(xs), up(w), up(s)
+    d_slots, d_pos = up(slots), up(positions)
+    q1, q2 = dev.DeviceBuffer(m * QKV * 2 + 16), dev.DeviceBuffer(m * QKV * 2)
+    st = up(np.zeros(1, np.int32))
+    kv.launch_paged_qkv_rope_append(dx, k_in, m, dw, ds, k_in, q1.ptr + 2 * q_off, pools[0][1], 1,
+                                    d_slots, d_pos, d_c, d_s, max_pos, NQ, d_status=st)
+    kv.launch_w8a16_gemm_batched(dx, k_in, m, dw, ds, q2, QKV, QKV, k_in)
+    plain = q2.download(np.uint16, (m, QKV))
+    kv.launch_paged_rope_append(q2, m, pools[1][1], 1, d_slots, d_pos, d_c, d_s, max_pos, NQ)
+    got = q1.download(np.uint16)[q_off:q_off + m * QKV].reshape(m, QKV)
+    want = q2.download(np.uint16, (m, QKV))
+    want[[7, m - 1]] = plain[[7, m - 1]]
+    assert np.array_equal(got, want)
+    assert np.array_equal(pools[0][0].download(np.uint8), pools[1][0].download(np.uint8))
+    assert st.download(np.int32, (1,))[0] == atomflow_amd.AF_ERR_OUT_OF_RANGE
