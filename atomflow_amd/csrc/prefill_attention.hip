@@ -11,12 +11,11 @@
 // kv_len = seq_kv is the reference's form (af_tiled_attention).
 //
 // Design: a workgroup is 4 waves of one Q head; each wave owns a block of 32
-// queries (128 queries per workgroup, two workgroups per CU, so each SIMD has a
-// second wave to issue matrix work during the other's softmax).
+// queries (128 queries per workgroup, two or three workgroups per CU, so each SIMD
+// has other waves to issue matrix work during one's softmax).
 //  * S^T = K Q^T on v_mfma_f32_32x32x16_f16: the A operand is a K fragment read
 //    from LDS, the B operand the query block held in registers for the whole
-//    launch (LDS delivers about 64 B/clk per CU, one 1 KB fragment per 16 clk;
-//    an MFMA takes 32).
+//    launch.
 //  * Each lane owns 16 of the 32 scores of one query (lane l^32 the other 16):
 //    the softmax is in-lane work plus one v_permlane32_swap.
 //  * O^T += V^T P^T. P^T is the S^T accumulator rounded to fp16: within each
@@ -25,19 +24,20 @@
 //    and the V^T operand is read with ds_read_b64_tr_b16 (a 16-lane group reads
 //    a 4-key x 16-d block and gets it transposed: lane l, element t = key t,
 //    d = l%16), two per operand.
-//  * K and V tiles of 64 keys are double-buffered in LDS, XOR-swizzled in 16-byte
-//    chunks (K by row%16 for the b128 operand reads, V by 4*(row%4) for the
-//    transposing reads). They go from global memory straight into LDS
-//    (global_load_lds_dwordx4, no registers); the next tile's loads are issued
-//    before the current tile's matrix work: one barrier per tile.
+//  * K and V tiles of 32 keys are kept two or four deep in LDS, XOR-swizzled in
+//    16-byte chunks (K by row%16 for the b128 operand reads, V by 4*(row%4) for
+//    the transposing reads). They go from global memory straight into LDS
+//    (lds_dma16, no registers); later tiles' loads are issued before the current
+//    tile's matrix work: one barrier per tile.
 //  * Softmax is online in the log2 domain with lazy rescaling: the running max
 //    moves only when a tile's probabilities sum past 2^8 in some lane, so most
 //    tiles skip both the tile max and the O^T rescale. The row sum is taken over
 //    the fp16 probabilities the P.V product uses.
-//  * Paged pools (PAGED): tile rows map through the sequence's block table; the
-//    entries for tile kt+1 are fetched during tile kt-1. FP8 pools (FP8) stage
-//    tiles through registers and convert E4M3 -> fp16 exactly on the way into
-//    LDS; the K scale joins the score scale and the V scale the output.
+//  * Paged pools (PAGED): the 8 rows a wave fetches of a tile lie in one block, so
+//    the block-table entry is a scalar load and the address scalar arithmetic.
+//    FP8 pools (FP8) stage tiles through registers and convert E4M3 -> fp16 exactly
+//    on the way into LDS; the K scale joins the score scale and the V scale the
+//    output.
 //  * Workgroups are ordered KV head fastest (consecutive workgroups alternate
 //    XCDs, so each XCD's L2 serves one KV head when n_kv_heads divides 8), then
 //    Q head, then query tile heaviest first; waves skip key tiles that lie wholly
@@ -63,8 +63,9 @@ namespace {
 constexpr int kPfHd = 128;
 constexpr int kPfWaves = 4;
 constexpr int kPfThreads = 64 * kPfWaves;
-constexpr int kPfKeys = 64;                      // keys per LDS tile
-constexpr int kTileBytes = kPfKeys * kPfHd * 2;  // one K or V tile: 64 rows of 256 B
+constexpr int kPfKeys = 64;                      // keys per planned key tile (splits, pieces)
+constexpr int kLdsKeys = 32;                     // keys per LDS tile
+constexpr int kTileBytes = kLdsKeys * kPfHd * 2;  // one K or V tile: rows of 256 B
 constexpr float kPfSumLimit = 256.0f;  // per-lane tile row sum that forces a rescale
 constexpr float kPfEmptyMax = -1e30f;
 constexpr int kPfQueries = 32 * kPfWaves;  // queries per workgroup (query tile)
@@ -158,74 +159,69 @@ __device__ __forceinline__ uint4 ld16(const uint16_t* p) {
     return *reinterpret_cast<const uint4*>(p);
 }
 
-// Loads one 64-key K or V tile straight into LDS (global_load_lds_dwordx4: lane
-// l of a wave writes the 16 bytes at LDS base + 16*l). Wave w fills rows
-// 16w .. 16w+15, four rows per instruction; the lane at physical chunk p of row r
-// fetches logical chunk p ^ swz(r), which realises the swizzled layout. Rows past
-// kv_len load row kv_len-1: finite data whose scores are masked. base: the
-// head's first element in cache row (slot) 0, as bytes. Contiguous caches use
-// 32-bit row offsets (scalar base + vector offset); paged pools map the row
-// through blk[i], the physical block of the lane's row in instruction i.
-template <bool IS_K, bool PAGED>
-__device__ __forceinline__ void dma_tile(const char* base, uint32_t row_bytes, int key0,
-                                         int kv_len, int wave, int lane, char* lds_tile,
-                                         const int (&blk)[4], int bs_log2, int max_block) {
+// Where a wave's 8 rows of a 32-key tile come from. Rows 8 wave .. 8 wave + 7 of a
+// tile start at a multiple of 8, so they lie in one block of a paged pool (block
+// sizes are powers of two >= 8): the block id and the first row's address are
+// scalar, and a lane adds its row and 16-byte chunk. Rows past kv_len read row
+// kv_len - 1: finite data whose scores are masked.
+struct RowSource {
+    int64_t row;  // cache row (slot) of the first of the 8
+    int last;     // index of the last row to read, 0 .. 7 (later rows repeat it)
+};
+// The block-table entry of the wave's rows of tile kt, as loaded (paged pools).
+template <bool PAGED>
+__device__ __forceinline__ int tile_entry(const PrefillArgs& a, int kt, int wave) {
+    if constexpr (!PAGED) return 0;
+    typedef const __attribute__((address_space(4))) int32_t* const_i32;  // a scalar load
+    return ((const_i32)(uintptr_t)a.table)[min(kt * kLdsKeys + 8 * wave, a.kv_len - 1) >> a.bs_log2];
+}
+template <bool PAGED>
+__device__ __forceinline__ RowSource tile_rows(const PrefillArgs& a, int kt, int wave, int entry) {
+    const int want = kt * kLdsKeys + 8 * wave;
+    const int key = min(want, a.kv_len - 1);
+    RowSource src;
+    src.last = min(7, max(0, a.kv_len - 1 - want));
+    src.row = key;
+    if constexpr (PAGED) {
+        const int blk = min(max(entry, 0), a.max_block);  // never address outside the pool
+        src.row = (int64_t(__builtin_amdgcn_readfirstlane(blk)) << a.bs_log2) |
+                  (key & ((1 << a.bs_log2) - 1));
+    }
+    return src;
+}
+
+// Loads the wave's 8 rows of one K or V tile straight into LDS: lane l of a wave
+// writes the 16 bytes at LDS base + 16 l, four rows per instruction; the lane at
+// physical chunk p of row r fetches logical chunk p ^ swz(r), which realises the
+// swizzled layout. base: the head's first element in cache row 0, as bytes.
+template <bool IS_K>
+__device__ __forceinline__ void dma_rows(const char* base, uint32_t row_bytes, const RowSource& src,
+                                         int wave, int lane, uint32_t lds_tile) {
+    const char* first = base + src.row * row_bytes;
     const int pr = lane >> 4, pc = lane & 15;
-    const uint32_t dst = lds_address(lds_tile) + 16 * wave * 256;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = 16 * wave + 4 * i + pr;  // tile row
+    for (int i = 0; i < 2; ++i) {
+        const int r = 8 * wave + 4 * i + pr;  // tile row
         const int chunk = IS_K ? (pc ^ (r & 15)) : (pc ^ (4 * (r & 3)));
-        const int key = min(key0 + r, kv_len - 1);
-        if constexpr (PAGED) {
-            const int b = min(max(blk[i], 0), max_block);  // never address outside the pool
-            const int64_t slot = (int64_t(b) << bs_log2) | (key & ((1 << bs_log2) - 1));
-            lds_dma16(base + slot * row_bytes + 16 * chunk, dst + 4 * i * 256);
-        } else {
-            lds_dma16(base, __umul24(uint32_t(key), row_bytes) + 16u * chunk, dst + 4 * i * 256);
-        }
+        lds_dma16(first, __umul24(uint32_t(min(4 * i + pr, src.last)), row_bytes) + 16u * chunk,
+                  lds_tile + (8 * wave + 4 * i) * 256);
     }
 }
 
-// Block-table entries of the rows this lane fetches for tile `kt` (paged pools),
-// as loaded: dma_tile clamps them to the pool when it uses them, a tile later.
-// (Clamped here, the wait for the entries would also wait for the tile DMA
-// issued just before them.)
-__device__ __forceinline__ void tile_blocks(const int32_t* table, int bs_log2, int kt, int kv_len,
-                                            int wave, int lane, int (&blk)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        blk[i] = table[min(kt * kPfKeys + 16 * wave + 4 * i + (lane >> 4), kv_len - 1) >> bs_log2];
-}
-
-// Block-table entry of logical row `key` (paged FP8 pools), as loaded: fp8_load
-// clamps it to the pool a tile later, for the same reason.
-__device__ __forceinline__ int table_entry(const PrefillArgs& a, int key) {
-    return a.table[key >> a.bs_log2];
-}
-
-// FP8 pools: tile rows go through registers, 32 codes of K and of V per thread
-// (row tid/4, elements 32*(tid%4) ..), converted to fp16 exactly (E4M3 -> fp16,
-// unit scale) after the current tile's matrix work and stored in the same
+// FP8 pools: tile rows go through registers, 16 codes of K and of V per thread
+// (row tid / 8, elements 16 (tid % 8) ..), converted to fp16 exactly (E4M3 ->
+// fp16, unit scale) after the current tile's matrix work and stored in the same
 // swizzled layout as the DMA path. The K/V scales are applied to the scores and
 // the output instead.
 struct Fp8Tile {
-    uint4 k0, k1, v0, v1;
+    uint4 k, v;
 };
 
-template <bool PAGED>
 __device__ __forceinline__ void fp8_load(const char* kb, const char* vb, uint32_t row_bytes,
-                                         int key0, int kv_len, int tid, int blk, int bs_log2,
-                                         int max_block, Fp8Tile& t) {
-    const int key = min(key0 + (tid >> 2), kv_len - 1);
-    const int b = min(max(blk, 0), max_block);  // never address outside the pool
-    const int64_t slot =
-        PAGED ? ((int64_t(b) << bs_log2) | (key & ((1 << bs_log2) - 1))) : int64_t(key);
-    const size_t off = size_t(slot) * row_bytes + 32 * (tid & 3);
-    t.k0 = *reinterpret_cast<const uint4*>(kb + off);
-    t.k1 = *reinterpret_cast<const uint4*>(kb + off + 16);
-    t.v0 = *reinterpret_cast<const uint4*>(vb + off);
-    t.v1 = *reinterpret_cast<const uint4*>(vb + off + 16);
+                                         const RowSource& src, int lane, Fp8Tile& t) {
+    const uint32_t off = __umul24(uint32_t(min(lane >> 3, src.last)), row_bytes) + 16u * (lane & 7);
+    t.k = *reinterpret_cast<const uint4*>(kb + src.row * row_bytes + off);
+    t.v = *reinterpret_cast<const uint4*>(vb + src.row * row_bytes + off);
 }
 
 // Eight E4M3 codes (two words) -> eight fp16 values.
@@ -239,25 +235,17 @@ __device__ __forceinline__ uint4 e4m3x8_to_f16(uint32_t w0, uint32_t w1) {
 }
 
 __device__ __forceinline__ void fp8_store(char* ks, char* vs, int tid, const Fp8Tile& t) {
-    const int row = tid >> 2, q = tid & 3;
-    // chunk 4q + c holds elements 32q + 8c .. +7
-    *reinterpret_cast<uint4*>(ks + k_off(row, 4 * q + 0)) = e4m3x8_to_f16(t.k0.x, t.k0.y);
-    *reinterpret_cast<uint4*>(ks + k_off(row, 4 * q + 1)) = e4m3x8_to_f16(t.k0.z, t.k0.w);
-    *reinterpret_cast<uint4*>(ks + k_off(row, 4 * q + 2)) = e4m3x8_to_f16(t.k1.x, t.k1.y);
-    *reinterpret_cast<uint4*>(ks + k_off(row, 4 * q + 3)) = e4m3x8_to_f16(t.k1.z, t.k1.w);
-    // V's swizzle permutes whole 64-B chunk groups by row % 4, so the same store
-    // of rows r and r + 1 would meet in the same banks (counters: 0.67 conflicts
-    // per LDS access). Each lane stores its four chunks rotated by row % 4, so
-    // one instruction's rows land in different 16-B bank groups.
-    const uint4 c0 = e4m3x8_to_f16(t.v0.x, t.v0.y), c1 = e4m3x8_to_f16(t.v0.z, t.v0.w);
-    const uint4 c2 = e4m3x8_to_f16(t.v1.x, t.v1.y), c3 = e4m3x8_to_f16(t.v1.z, t.v1.w);
-    const int rot = row & 3;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int cc = (c + rot) & 3;
-        const uint4 val = cc == 0 ? c0 : cc == 1 ? c1 : cc == 2 ? c2 : c3;
-        *reinterpret_cast<uint4*>(vs + v_off(row, 4 * q + cc)) = val;
-    }
+    const int row = tid >> 3, q = tid & 7;
+    // chunk 2q + c holds elements 16q + 8c .. +7. K's swizzle puts the even
+    // chunks of adjacent rows in different banks; V's keeps a chunk's parity, so
+    // odd rows store their odd chunk first.
+    *reinterpret_cast<uint4*>(ks + k_off(row, 2 * q)) = e4m3x8_to_f16(t.k.x, t.k.y);
+    *reinterpret_cast<uint4*>(ks + k_off(row, 2 * q + 1)) = e4m3x8_to_f16(t.k.z, t.k.w);
+    const bool odd = row & 1;
+    const uint32_t a0 = odd ? t.v.z : t.v.x, a1 = odd ? t.v.w : t.v.y;
+    const uint32_t b0 = odd ? t.v.x : t.v.z, b1 = odd ? t.v.y : t.v.w;
+    *reinterpret_cast<uint4*>(vs + v_off(row, 2 * q + (odd ? 1 : 0))) = e4m3x8_to_f16(a0, a1);
+    *reinterpret_cast<uint4*>(vs + v_off(row, 2 * q + (odd ? 0 : 1))) = e4m3x8_to_f16(b0, b1);
 }
 
 __device__ __forceinline__ half8 lds_half8(const char* p) {
@@ -304,8 +292,6 @@ __device__ __forceinline__ float dot2_sum(const half8& h, float acc) {
     return acc;
 }
 
-// LDS: K tiles at [0, 2*kTileBytes), V tiles after them.
-constexpr int kVBase = 2 * kTileBytes;
 
 __device__ __forceinline__ void store_agent2(uint64_t* p, float x, float y) {
     const auto u = [](float f) { return uint64_t(__builtin_bit_cast(uint32_t, f)); };
@@ -430,11 +416,23 @@ __device__ __forceinline__ void merge_pieces(const PrefillArgs& a, float16v (&o)
     }
 }
 
-template <bool PAGED, bool FP8>
-__global__ __launch_bounds__(kPfThreads, 2) void prefill_attention_kernel(const PrefillArgs args) {
+// DEEP: the scores of tile t + 1 are taken beside the softmax of tile t and every
+// operand is read before the math that needs it, over four LDS tiles and up to
+// 256 VGPRs (two workgroups per CU). Otherwise a step is one tile from scores to
+// P.V over two LDS tiles, in 168 VGPRs (three workgroups per CU, whose waves cover
+// each other). Both do the same arithmetic in the same order. Launches of few
+// workgroups are bound by a wave's own chain and take DEEP; long ones by the
+// card's power (the clock falls to 1.5 GHz as the matrix cores fill), where the
+// plain form spends less (us, DEEP / plain / the former 64-key tiles with two
+// workgroups per CU: 4096-token prompt 113 / 119 / 123, 2048 tokens behind 6144
+// 203 / 215 / 211, 8192-token prompt 416 / 404 / 444, 16384 1585 / 1521 / 1711).
+template <bool PAGED, bool FP8, bool DEEP>
+__global__ __launch_bounds__(kPfThreads, DEEP ? 2 : 3) void prefill_attention_kernel(const PrefillArgs args) {
     PrefillArgs a = args;
     constexpr int kQueries = 32 * kPfWaves;  // per workgroup
-    __shared__ __align__(16) char s_lds[4 * kTileBytes];
+    constexpr int kStages = DEEP ? 4 : 2;        // LDS tiles of K, then of V
+    constexpr int kVBase = kStages * kTileBytes;
+    __shared__ __align__(16) char s_lds[2 * kStages * kTileBytes];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -507,6 +505,9 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_attention_kernel(const 
         kt_lo = piece * all / pieces;
         n_kt = (piece + 1) * all / pieces;
     }
+    // From here on in LDS tiles.
+    kt_lo *= kPfKeys / kLdsKeys;
+    n_kt = min(n_kt * (kPfKeys / kLdsKeys), (wg_keys + kLdsKeys - 1) / kLdsKeys);
     // Keys the wave needs.
     const int w_keys = wave_live ? min(a.p0 + min(wq0 + 32, a.n), a.kv_len) : 0;
 
@@ -542,36 +543,36 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_attention_kernel(const 
 #pragma unroll
         for (int s = 0; s < 8; ++s) qf[s] = __builtin_bit_cast(half8, ld16(qrow + 16 * s));
     }
-    // Keep the query loads ahead of the tile loads: the prologue's wait for the
-    // tile then covers them, and the loop never waits on a query register.
-    asm volatile("" ::: "memory");
     constexpr int kElem = FP8 ? 1 : 2;
     const char* kb = reinterpret_cast<const char*>(a.k) + size_t(kvh) * kPfHd * kElem;
     const char* vb = reinterpret_cast<const char*>(a.v) + size_t(kvh) * kPfHd * kElem;
-    // Paged: the block-table entries of tile kt+1 are loaded one step ahead, so
-    // the wait for tile kt's data also covers them.
-    int blk[4] = {0, 0, 0, 0};
-    int blk8 = 0;  // FP8: this thread's row's block for the next tile
+    const uint32_t lds0 = lds_address(s_lds);
     Fp8Tile f8;
-    const int key_lo = kt_lo * kPfKeys;
-    if constexpr (FP8) {
-        if constexpr (PAGED) blk8 = table_entry(a, min(key_lo + (tid >> 2), a.kv_len - 1));
-        fp8_load<PAGED>(kb, vb, a.kv_row_bytes, key_lo, a.kv_len, tid, blk8, a.bs_log2,
-                        a.max_block, f8);
-        fp8_store(s_lds, s_lds + kVBase, tid, f8);
-        if constexpr (PAGED)
-            if (kt_lo + 1 < n_kt)
-                blk8 = table_entry(a, min(key_lo + kPfKeys + (tid >> 2), a.kv_len - 1));
-    } else {
-        if constexpr (PAGED)
-            tile_blocks(a.table, a.bs_log2, kt_lo, a.kv_len, wave, lane, blk);
-        dma_tile<true, PAGED>(kb, a.kv_row_bytes, key_lo, a.kv_len, wave, lane, s_lds, blk,
-                              a.bs_log2, a.max_block);
-        dma_tile<false, PAGED>(vb, a.kv_row_bytes, key_lo, a.kv_len, wave, lane, s_lds + kVBase,
-                               blk, a.bs_log2, a.max_block);
-        if constexpr (PAGED)
-            if (kt_lo + 1 < n_kt)
-                tile_blocks(a.table, a.bs_log2, kt_lo + 1, a.kv_len, wave, lane, blk);
+    // Fetches tile kt: into `stage` (fp16), or into f8 for fp8_store. The plain
+    // form reads the block-table entry a step ahead; DEEP reads it here: with a
+    // scalar load outstanding, every wait for an LDS operand waits for all of
+    // them (five 512-token chunks with their projection 212 us, a step ahead 219).
+    int entry = DEEP ? 0 : tile_entry<PAGED>(a, kt_lo, wave);
+    auto fetch = [&](int kt, int stage) __attribute__((always_inline)) {
+        const RowSource src =
+            tile_rows<PAGED>(a, kt, wave, DEEP ? tile_entry<PAGED>(a, kt, wave) : entry);
+        if constexpr (FP8) {
+            fp8_load(kb, vb, a.kv_row_bytes, src, lane, f8);
+        } else {
+            dma_rows<true>(kb, a.kv_row_bytes, src, wave, lane, lds0 + stage * kTileBytes);
+            dma_rows<false>(vb, a.kv_row_bytes, src, wave, lane,
+                            lds0 + kVBase + stage * kTileBytes);
+        }
+    };
+    constexpr int kAhead = kStages - 1;  // tiles fetched ahead of the current one
+#pragma unroll
+    for (int i = 0; i < (DEEP ? kAhead : 1); ++i) {
+        if (kt_lo + i < n_kt) {
+            fetch(kt_lo + i, i);
+            if constexpr (FP8)
+                fp8_store(s_lds + i * kTileBytes, s_lds + kVBase + i * kTileBytes, tid, f8);
+        }
+        if constexpr (!DEEP) entry = tile_entry<PAGED>(a, min(kt_lo + 1, n_kt - 1), wave);
     }
     if (a.cos_t) {  // packed partials with RoPE (wave-uniform)
         // Whole 32-bit words in and out: two fp16 elements per word, low half
@@ -633,108 +634,157 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_attention_kernel(const 
     const float sc = FP8 ? a.scale_log2 * a.scales[kvh] : a.scale_log2;
     const float v_scale = FP8 ? a.scales[a.n_kv_heads + kvh] : 1.0f;
 
-    auto step = [&](int kt, auto buf_c) {
-        constexpr int BUF = decltype(buf_c)::value;
-        // This wave's tile loads have landed in LDS; the barrier covers the others'
-        // and frees the other buffer (read in the previous step) for the next tile.
-        lds_dma_wait();
-        __syncthreads();
-        if (kt + 1 < n_kt) {
-            if constexpr (FP8) {
-                fp8_load<PAGED>(kb, vb, a.kv_row_bytes, (kt + 1) * kPfKeys, a.kv_len, tid, blk8,
-                                a.bs_log2, a.max_block, f8);
-                if constexpr (PAGED)
-                    if (kt + 2 < n_kt)
-                        blk8 = table_entry(a, min((kt + 2) * kPfKeys + (tid >> 2), a.kv_len - 1));
-            } else {
-                dma_tile<true, PAGED>(kb, a.kv_row_bytes, (kt + 1) * kPfKeys, a.kv_len, wave, lane,
-                                      s_lds + (BUF ^ 1) * kTileBytes, blk, a.bs_log2,
-                                      a.max_block);
-                dma_tile<false, PAGED>(vb, a.kv_row_bytes, (kt + 1) * kPfKeys, a.kv_len, wave,
-                                       lane, s_lds + kVBase + (BUF ^ 1) * kTileBytes, blk,
-                                       a.bs_log2, a.max_block);
-                if constexpr (PAGED)
-                    if (kt + 2 < n_kt)
-                        tile_blocks(a.table, a.bs_log2, kt + 2, a.kv_len, wave, lane,
-                                    blk);
-            }
-        }
-        const int key0 = kt * kPfKeys;
-        const char* ks = s_lds + BUF * kTileBytes;
-        const char* vs = s_lds + BUF * kTileBytes;  // va[] carries the V region's base
-        // Two halves of 32 keys: QK^T, softmax, then P.V for each.
+    // Hides the keys of tile kt that this lane's query does not attend. Register r
+    // holds key 32 kt + 8(r/4) + 4hi + r%4.
+    auto mask_scores = [&](int kt, float16v& s) __attribute__((always_inline)) {
+        const int key0 = kt * kLdsKeys;
+        if (key0 + 32 <= mask_from) return;
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            const int keyh = key0 + 32 * kb;
-            if (keyh >= w_keys) break;  // wave-uniform
-            float16v sacc;
+        for (int r = 0; r < 16; ++r) {
+            const int key = key0 + 8 * (r >> 2) + 4 * hi + (r & 3);
+            s[r] = key < lim ? s[r] : -INFINITY;
+        }
+    };
+    // Probabilities against the running max m_run, rounded to fp16, and their row
+    // sum. While each lane's sum stays <= 2^8, every p is <= 2^8 and m_run is kept
+    // (it may trail the true max by up to 8 in log2 units; fp16 holds p to 2^15).
+    // Otherwise (the first keys, or scores that grew) the exact running max is
+    // taken and O^T, l rescaled: the max is computed only on this path.
+    auto softmax = [&](const float16v& s, half8 (&pj)[2]) __attribute__((always_inline)) {
+        float ls;
+        auto probs = [&]() __attribute__((always_inline)) {
+            float16v pv;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) pv[r] = fast_exp2(fmaf(s[r], sc, -m_run));
+            pj[0] = to_half8(pv, 0);
+            pj[1] = to_half8(pv, 8);
+            ls = dot2_sum(pj[1], dot2_sum(pj[0], 0.0f));
+        };
+        probs();
+        if (__builtin_amdgcn_ballot_w64(!(ls <= kPfSumLimit))) {
+            float mx = s[0];
+#pragma unroll
+            for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+            const float m_new = fmaxf(m_run, halves_max(mx) * sc);
+            const float alpha = fast_exp2(m_run - m_new);
+            m_run = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+            probs();
+        }
+        l_run += ls;
+    };
+    auto value_operand = [&](int stage, int jj, int db) __attribute__((always_inline)) {
+        const char* p = s_lds + stage * kTileBytes + va[db] + 16 * jj * 256;  // va[]: the V region
+        return lds_vt(p, p + 8 * 256);
+    };
+    // Tile kt + kAhead goes to the stage that the barrier before has freed.
+    auto fetch_ahead = [&](int kt, int stage) __attribute__((always_inline)) {
+        if (kt + kAhead < n_kt) fetch(kt + kAhead, stage);
+    };
+    auto end_step = [&](int kt, int stage) __attribute__((always_inline)) {
+        if constexpr (FP8)
+            if (kt + kAhead < n_kt)
+                fp8_store(s_lds + stage * kTileBytes, s_lds + kVBase + stage * kTileBytes, tid, f8);
+        if constexpr (PAGED && !DEEP) entry = tile_entry<PAGED>(a, min(kt + 2, n_kt - 1), wave);
+    };
+
+    if constexpr (!DEEP) {
+        auto step = [&](int kt, auto stage_c) __attribute__((always_inline)) {
+            constexpr int S = decltype(stage_c)::value;
+            // This wave's tile loads have landed in LDS; the barrier covers the
+            // others' and frees the other stage (read in the previous step).
+            lds_dma_wait();
+            __syncthreads();
+            fetch_ahead(kt, S ^ 1);
+            if (kt * kLdsKeys < w_keys) {  // wave-uniform
+                const char* ks = s_lds + S * kTileBytes;
+                float16v sacc;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sacc[r] = 0.0f;
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(lds_half8(ks + ka[s]), qf[s],
+                                                                  sacc, 0, 0, 0);
+                mask_scores(kt, sacc);
+                half8 pj[2];
+                softmax(sacc, pj);
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+                    for (int db = 0; db < 4; ++db)
+                        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(value_operand(S, jj, db),
+                                                                       pj[jj], o[db], 0, 0, 0);
+            }
+            end_step(kt, S ^ 1);
+        };
+        int kt = kt_lo;
+        for (; kt + 2 <= n_kt; kt += 2) {
+            step(kt, std::integral_constant<int, 0>{});
+            step(kt + 1, std::integral_constant<int, 1>{});
+        }
+        if (kt < n_kt) step(kt, std::integral_constant<int, 0>{});
+    } else {
+        auto scores = [&](int stage, float16v& sacc) __attribute__((always_inline)) {
+            const char* ks = s_lds + stage * kTileBytes;
+            half8 kf[8];
+#pragma unroll
+            for (int s = 0; s < 8; ++s) kf[s] = lds_half8(ks + ka[s]);
 #pragma unroll
             for (int r = 0; r < 16; ++r) sacc[r] = 0.0f;
 #pragma unroll
-            for (int s = 0; s < 8; ++s) {
-                const half8 kf = lds_half8(ks + ka[s] + kb * 32 * 256);
-                sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[s], sacc, 0, 0, 0);
+            for (int s = 0; s < 8; ++s)
+                sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s], qf[s], sacc, 0, 0, 0);
+        };
+        // Step kt: tile kt's softmax beside tile kt + 1's scores, then tile kt's P.V.
+        auto step = [&](int kt, auto stage_c, float16v& now, float16v& next)
+            __attribute__((always_inline)) {
+            constexpr int S = decltype(stage_c)::value;
+            // Tile kt + 1 has landed (tile kt + 2's loads may be in flight); the
+            // barrier covers the other waves' and frees tile kt - 1's stage.
+            if (!FP8 && kt + 2 < n_kt) wait_vmcnt<4>();
+            else if (!FP8) wait_vmcnt<0>();
+            __syncthreads();
+            fetch_ahead(kt, (S + 3) % kStages);
+            if (kt * kLdsKeys < w_keys) {  // wave-uniform
+                half8 vf[2][4];
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+                    for (int db = 0; db < 4; ++db) vf[jj][db] = value_operand(S, jj, db);
+                mask_scores(kt, now);
+                // (past the last tile: whatever the stage holds, unused)
+                scores((S + 1) % kStages, next);
+                half8 pj[2];
+                softmax(now, pj);
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+                    for (int db = 0; db < 4; ++db)
+                        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[jj][db], pj[jj], o[db], 0,
+                                                                       0, 0);
             }
-            // Register r holds key keyh + 8(r/4) + 4hi + r%4.
-            if (keyh + 32 > mask_from) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = keyh + 8 * (r >> 2) + 4 * hi + (r & 3);
-                    sacc[r] = key < lim ? sacc[r] : -INFINITY;
-                }
-            }
-            // Probabilities against the running max m_run, rounded to fp16, and
-            // their row sum. While each lane's sum stays <= 2^8, every p is <= 2^8
-            // and m_run is kept (it may trail the true max by up to 8 in log2
-            // units; fp16 holds p to 2^15). Otherwise (the first keys, or scores
-            // that grew) the exact running max is taken and O^T, l rescaled: the
-            // max is computed only on this path.
-            half8 pj[2];
-            float ls;
-            auto probs = [&]() {
-                float16v pv;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) pv[r] = fast_exp2(fmaf(sacc[r], sc, -m_run));
-                pj[0] = to_half8(pv, 0);
-                pj[1] = to_half8(pv, 8);
-                ls = dot2_sum(pj[1], dot2_sum(pj[0], 0.0f));
-            };
-            probs();
-            if (__builtin_amdgcn_ballot_w64(!(ls <= kPfSumLimit))) {
-                float mx = sacc[0];
-#pragma unroll
-                for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sacc[r]);
-                const float m_new = fmaxf(m_run, halves_max(mx) * sc);
-                const float alpha = fast_exp2(m_run - m_new);
-                m_run = m_new;
-                l_run *= alpha;
-#pragma unroll
-                for (int db = 0; db < 4; ++db)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-                probs();
-            }
-            l_run += ls;
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                for (int db = 0; db < 4; ++db) {
-                    const char* p = vs + va[db] + 16 * (2 * kb + jj) * 256;
-                    const half8 vt = lds_vt(p, p + 8 * 256);
-                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vt, pj[jj], o[db], 0, 0, 0);
-                }
+            end_step(kt, (S + 3) % kStages);
+        };
+        lds_dma_wait();
+        __syncthreads();
+        float16v s0, s1;
+        scores(0, s0);
+        int kt = kt_lo;
+        for (;;) {
+            step(kt, std::integral_constant<int, 0>{}, s0, s1);
+            if (++kt >= n_kt) break;
+            step(kt, std::integral_constant<int, 1>{}, s1, s0);
+            if (++kt >= n_kt) break;
+            step(kt, std::integral_constant<int, 2>{}, s0, s1);
+            if (++kt >= n_kt) break;
+            step(kt, std::integral_constant<int, 3>{}, s1, s0);
+            if (++kt >= n_kt) break;
         }
-        if constexpr (FP8)
-            if (kt + 1 < n_kt)
-                fp8_store(s_lds + (BUF ^ 1) * kTileBytes, s_lds + kVBase + (BUF ^ 1) * kTileBytes,
-                          tid, f8);
-    };
-    int kt = kt_lo;
-    for (; kt + 2 <= n_kt; kt += 2) {
-        step(kt, std::integral_constant<int, 0>{});
-        step(kt + 1, std::integral_constant<int, 1>{});
     }
-    if (kt < n_kt) step(kt, std::integral_constant<int, 0>{});
 
     if (pieces > 1) {
         merge_pieces(a, o, m_run, l_run, rec_tile, head, piece, pieces, t0, wq0, wave_live, v_scale);
@@ -778,17 +828,28 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_attention_kernel(const 
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-int launch_prefill(PrefillArgs a, hipStream_t stream) {
-    a.n_tiles = ceil_div(a.n, 32 * kPfWaves);
-    const dim3 grid(a.n_tiles * a.n_q_heads * std::max(a.n_pieces, 1)), block(kPfThreads);
+// Launches `wgs` workgroups: FP8 pools always DEEP, fp16 up to about four
+// workgroups per CU (see the kernel).
+int launch_grid(const PrefillArgs& a, int wgs, hipStream_t stream) {
+    const dim3 grid(wgs), block(kPfThreads);
+    const bool deep = wgs <= 4 * device_compute_units();
     if (a.scales)
-        hipLaunchKernelGGL((prefill_attention_kernel<true, true>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((prefill_attention_kernel<true, true, true>), grid, block, 0, stream, a);
+    else if (a.table && deep)
+        hipLaunchKernelGGL((prefill_attention_kernel<true, false, true>), grid, block, 0, stream, a);
     else if (a.table)
-        hipLaunchKernelGGL((prefill_attention_kernel<true, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((prefill_attention_kernel<true, false, false>), grid, block, 0, stream, a);
+    else if (deep)
+        hipLaunchKernelGGL((prefill_attention_kernel<false, false, true>), grid, block, 0, stream, a);
     else
-        hipLaunchKernelGGL((prefill_attention_kernel<false, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((prefill_attention_kernel<false, false, false>), grid, block, 0, stream, a);
     AF_TRY_LAUNCH();
     return AF_OK;
+}
+
+int launch_prefill(PrefillArgs a, hipStream_t stream) {
+    a.n_tiles = ceil_div(a.n, 32 * kPfWaves);
+    return launch_grid(a, a.n_tiles * a.n_q_heads * std::max(a.n_pieces, 1), stream);
 }
 
 }  // namespace
@@ -825,13 +886,7 @@ int launch_prefix_partials(const PrefixPartialArgs& p, hipStream_t stream) {
     a.sin_t = p.sin_t;
     a.positions = p.positions;
     a.max_pos = p.max_pos;
-    const dim3 grid(a.n_tiles * a.n_q_heads * p.key_splits), block(kPfThreads);
-    if (p.scales)
-        hipLaunchKernelGGL((prefill_attention_kernel<true, true>), grid, block, 0, stream, a);
-    else
-        hipLaunchKernelGGL((prefill_attention_kernel<true, false>), grid, block, 0, stream, a);
-    AF_TRY_LAUNCH();
-    return AF_OK;
+    return launch_grid(a, a.n_tiles * a.n_q_heads * p.key_splits, stream);
 }
 
 // Key-tiles per piece for a launch whose query tiles need units[i] 64-key
@@ -1206,14 +1261,7 @@ static int prefill_batched(const void* q, int q_stride, const af_kv_pool* pool, 
             carve_records(a, workspace, n_groups, max_pieces);
         }
     }
-    const dim3 grid(n_tiles * n_q_heads), block(kPfThreads);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (fp8)
-        hipLaunchKernelGGL((prefill_attention_kernel<true, true>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((prefill_attention_kernel<true, false>), grid, block, 0, s, a);
-    AF_TRY_LAUNCH();
-    return AF_OK;
+    return launch_grid(a, n_tiles * n_q_heads, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int af_paged_prefill_attention_batched(

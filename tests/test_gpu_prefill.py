@@ -342,6 +342,44 @@ def test_paged_prefill_attention_vs_oracle(gpu, bs, p0, n, kv_len):
                                                     threads=8), what="vs fp32 oracle")
 
 
+@pytest.mark.parametrize("bs,p0,kv_len", [(8, 0, 5600), (32, 77, 5641)])
+def test_prefill_forms_give_the_same_bits(gpu, bs, p0, kv_len):
+    """A launch of more than four workgroups per CU (5600 queries x 24 heads) and
+    launches of few take different loops over the same arithmetic, and a paged pool
+    other addresses: contiguous, paged, and the chunk's first 1000 and last 37
+    queries launched alone give the same bits (kv_len inside the last 32 keys'
+    tile; blocks of 8 rows, the fewest a pool allows)."""
+    n = 5600
+    say(f"prefill forms bs={bs} p0={p0} n={n} kv_len={kv_len}")
+    max_blocks = (kv_len + bs - 1) // bs
+    nblocks = max_blocks + 3
+    host, buf, pool = _paged_pool(bs, nblocks, 1, 0xA70F78 + bs)
+    table = rng(bs).permutation(nblocks)[:max_blocks].astype(np.int32)
+    kc = oracle.paged_gather(host[0, 0], table, kv_len, bs, KV_DIM)
+    vc = oracle.paged_gather(host[0, 1], table, kv_len, bs, KV_DIM)
+    q = randn_f16((n, Q_DIM), 0xA70F79)
+    d_q, d_k, d_v, d_t = up(q), up(kc), up(vc), up(table)
+    outs = [dev.DeviceBuffer(n * Q_DIM * 2) for _ in range(3)]
+    kv.launch_prefill_attention(d_q, Q_DIM, d_k, d_v, outs[0], Q_DIM, p0, n, kv_len, kv_len, NQ,
+                                NKV, HD)
+    kv.launch_paged_prefill_attention(d_q, Q_DIM, pool, 0, d_t, max_blocks, p0, n, kv_len, outs[1],
+                                      Q_DIM, NQ)
+    want = outs[0].download(np.uint16, (n, Q_DIM))
+    assert np.all(np.isfinite(want.view(np.float16)))
+    assert np.array_equal(outs[1].download(np.uint16, (n, Q_DIM)), want)
+    for first, rows in ((0, 1000), (n - 37, 37)):
+        off = first * Q_DIM * 2
+        for paged in (False, True):
+            if paged:
+                kv.launch_paged_prefill_attention(d_q.ptr + off, Q_DIM, pool, 0, d_t, max_blocks,
+                                                  p0 + first, rows, kv_len, outs[2], Q_DIM, NQ)
+            else:
+                kv.launch_prefill_attention(d_q.ptr + off, Q_DIM, d_k, d_v, outs[2], Q_DIM,
+                                            p0 + first, rows, kv_len, kv_len, NQ, NKV, HD)
+            got = outs[2].download(np.uint16)[:rows * Q_DIM].reshape(rows, Q_DIM)
+            assert np.array_equal(got, want[first:first + rows]), (first, rows, paged)
+
+
 def test_paged_prefill_rejects_bad_arguments(gpu):
     say("paged prefill argument checks")
     lib = atomflow_amd.lib()
