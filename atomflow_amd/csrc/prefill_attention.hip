@@ -427,7 +427,7 @@ __device__ __forceinline__ void merge_pieces(const PrefillArgs& a, float16v (&o)
 // workgroups per CU: 4096-token prompt 113 / 119 / 123, 2048 tokens behind 6144
 // 203 / 215 / 211, 8192-token prompt 416 / 404 / 444, 16384 1585 / 1521 / 1711).
 template <bool PAGED, bool FP8, bool DEEP>
-__global__ __launch_bounds__(kPfThreads, DEEP ? 2 : 3) void prefill_attention_kernel(const PrefillArgs args) {
+__device__ __forceinline__ void prefill_body(const PrefillArgs& args) {
     PrefillArgs a = args;
     constexpr int kQueries = 32 * kPfWaves;  // per workgroup
     constexpr int kStages = DEEP ? 4 : 2;        // LDS tiles of K, then of V
@@ -826,6 +826,18 @@ __global__ __launch_bounds__(kPfThreads, DEEP ? 2 : 3) void prefill_attention_ke
         }
 }
 
+// The plain form (FP8 pools: DEEP always).
+template <bool PAGED, bool FP8>
+__global__ __launch_bounds__(kPfThreads, FP8 ? 2 : 3) void prefill_attention_kernel(
+    const PrefillArgs a) {
+    prefill_body<PAGED, FP8, FP8>(a);
+}
+
+template <bool PAGED>
+__global__ __launch_bounds__(kPfThreads, 2) void prefill_deep_kernel(const PrefillArgs a) {
+    prefill_body<PAGED, false, true>(a);
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Launches `wgs` workgroups: FP8 pools always DEEP, fp16 up to about four
@@ -834,15 +846,15 @@ int launch_grid(const PrefillArgs& a, int wgs, hipStream_t stream) {
     const dim3 grid(wgs), block(kPfThreads);
     const bool deep = wgs <= 4 * device_compute_units();
     if (a.scales)
-        hipLaunchKernelGGL((prefill_attention_kernel<true, true, true>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((prefill_attention_kernel<true, true>), grid, block, 0, stream, a);
     else if (a.table && deep)
-        hipLaunchKernelGGL((prefill_attention_kernel<true, false, true>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((prefill_deep_kernel<true>), grid, block, 0, stream, a);
     else if (a.table)
-        hipLaunchKernelGGL((prefill_attention_kernel<true, false, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((prefill_attention_kernel<true, false>), grid, block, 0, stream, a);
     else if (deep)
-        hipLaunchKernelGGL((prefill_attention_kernel<false, false, true>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((prefill_deep_kernel<false>), grid, block, 0, stream, a);
     else
-        hipLaunchKernelGGL((prefill_attention_kernel<false, false, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((prefill_attention_kernel<false, false>), grid, block, 0, stream, a);
     AF_TRY_LAUNCH();
     return AF_OK;
 }

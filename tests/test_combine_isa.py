@@ -188,6 +188,46 @@ def test_prefill_key_piece_publication_order(tmp_path):
 
 @pytest.mark.skipif(not os.path.exists(HIPCC) and shutil.which("hipcc") is None,
                     reason="hipcc not available")
+def test_prefill_deep_publication_and_prefetch(tmp_path):
+    """The software-pipelined prefill kernels publish key pieces in the same order,
+    and no prefill kernel waits for all vector memory between a tile's DMA and its
+    first matrix instruction (the tile is used a step or more later)."""
+    r, out = _compile(tmp_path, src="prefill_attention")
+    assert r.returncode == 0, r.stderr[-2000:]
+    asm = open(out).read()
+    checked = 0
+    for name, ins in _functions(asm, "prefill_deep_kernel"):
+        a, = [i for i, l in enumerate(ins) if l.startswith("global_atomic")]
+        bar = max(i for i in range(a) if ins[i].startswith("s_barrier"))
+        wait = max(i for i in range(bar) if ins[i].startswith("s_waitcnt") and
+                   ("vmcnt(0)" in ins[i] or ins[i] == "s_waitcnt 0"))
+        assert not any(l.startswith(("global_", "buffer_", "flat_")) for l in ins[wait + 1:a])
+        stores = [i for i, l in enumerate(ins) if l.startswith("global_store") and " sc1" in l]
+        assert len([i for i in stores if i < wait]) >= 32 + 2, name
+        loads = [i for i, l in enumerate(ins) if l.startswith("global_load") and " sc1" in l]
+        assert loads and min(loads) > a, name
+        checked += 1
+    assert checked == 2, checked  # contiguous, paged fp16
+    for kernel in ("prefill_deep_kernel", "prefill_attention_kernel"):
+        for name, ins in _functions(asm, kernel):
+            dma = [i for i, l in enumerate(ins) if l.startswith("global_load_lds")]
+            mfma = [i for i, l in enumerate(ins) if l.startswith("v_mfma")]
+            steps = 0
+            for i in dma:
+                # the last DMA of a tile inside the loop: a matrix instruction
+                # follows before the next barrier
+                nxt = min((m for m in mfma if m > i), default=None)
+                if nxt is None or any(ins[j].startswith(("s_barrier", "global_load_lds"))
+                                      for j in range(i + 1, nxt)):
+                    continue
+                assert not any(ins[j].startswith("s_waitcnt") and "vmcnt" in ins[j]
+                               for j in range(i + 1, nxt)), (name, ins[i:nxt])
+                steps += 1
+            assert steps >= 2 or not dma, (name, steps)
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC) and shutil.which("hipcc") is None,
+                    reason="hipcc not available")
 def test_kv_rows_load_policy(decode_asm):
     """Decode kernels read KV rows with non-temporal 16-byte loads (`global_load_dwordx4 ...
     nt`), except the CACHED instantiations (pools with AF_KV_POOL_SHARED_BLOCKS), which use no
