@@ -158,6 +158,10 @@ struct AttnArgs {
     int32_t n_kv_heads;
     int32_t num_splits;
     int32_t span_tokens;  // target tokens per split: a sequence uses ceil(L / span) splits
+    // Compact grid of up to 64 sequences, target_splits > 0: every sequence's span
+    // is the smallest (at least kMinSpan, at most span_tokens) with which the
+    // batch has at most target_splits splits (see adaptive_span).
+    int32_t target_splits;
     float qk_scale;       // log2(e) / sqrt(head_dim)
     const float* scales;  // FP8: [2][n_kv_heads] (K, V) of this layer
     float* part_o;        // [batch][n_kv_heads][rec_stride][GROUP * head_dim]
@@ -406,19 +410,6 @@ __device__ __forceinline__ void block_exclusive_scan(const int32_t* v, int64_t* 
     __syncthreads();
 }
 
-// Splits of a sequence attending L rows in the grid form (rows of STEP per
-// workgroup step): the rows after the shared prefix (all rows [0, L) when L is
-// below it) in spans of about span_tokens, at least one and at most
-// num_splits; an empty sequence keeps one workgroup for its zero output.
-__device__ __forceinline__ int grid_splits(const AttnArgs& a, int L, int step_rows) {
-    if (L <= 0) return 1;
-    const bool below_prefix = L < a.row_start;
-    const int t_lo = below_prefix ? 0 : min(a.row_start, L - 1);
-    const int total_steps = (L - t_lo + step_rows - 1) / step_rows;
-    const int span_steps = max(1, a.span_tokens / step_rows);
-    return max(1, min(a.num_splits, (total_steps + span_steps - 1) / span_steps));
-}
-
 // Inclusive prefix sum over the wave's 64 lanes on DPP: row_shr 1, 2, 4, 8
 // within each 16-lane row, then row_bcast 15 and 31 carry the row totals up.
 __device__ __forceinline__ int wave_inclusive_sum(int x) {
@@ -429,6 +420,68 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
     x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false); // row_bcast:15 -> rows 1, 3
     x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false); // row_bcast:31 -> rows 2, 3
     return x;
+}
+
+// Inclusive prefix maximum of non-negative values, the same way.
+__device__ __forceinline__ int wave_inclusive_max(int x) {
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
+    return x;
+}
+
+// Splits of a sequence attending L rows in the grid form (rows of STEP per
+// workgroup step): the rows after the shared prefix (all rows [0, L) when L is
+// below it) in spans of about span_steps, at least one and at most num_splits; an
+// empty sequence keeps one workgroup for its zero output.
+__device__ __forceinline__ int grid_splits(const AttnArgs& a, int L, int step_rows,
+                                           int span_steps) {
+    if (L <= 0) return 1;
+    const bool below_prefix = L < a.row_start;
+    const int t_lo = below_prefix ? 0 : min(a.row_start, L - 1);
+    const int total_steps = (L - t_lo + step_rows - 1) / step_rows;
+    return max(1, min(a.num_splits, (total_steps + span_steps - 1) / span_steps));
+}
+
+// Span of a small batch, in workgroup steps; lane s holds sequence s's length L
+// (any value past the batch). Wave-uniform. A launch whose (sequence, head) pairs
+// are few can give every split a CU of its own, and it ends with its longest
+// split: the span that spreads the batch's rows over target_splits splits is best
+// as long as no CU gets a second workgroup. Rounding each sequence up adds splits,
+// so the target is lowered by what the count overshoots; with the last attempt,
+// all / (target - batch), it cannot. When no length is more than 1/8 above the
+// mean, all sequences take the same number of splits: there a few rows more would
+// give some sequences one split more than the others (3 sequences of 30000 ..
+// 32768 fp16 rows 73.3 us, with the general search 73.9; 8 FP8 ones of 12000 ..
+// 12288 50.5 and 51.0). (us on MI355X, QKV projection included, 24
+// query and 8 KV heads, one split count for all sequences / these spans: 8
+// sequences of 768 .. 12288 rows 57.7 / 49.4 fp16 and 71.0 / 38.0 FP8, 12 of 256
+// .. 4096 40.9 / 33.1 and 54.8 / 30.3, 15 of 512 .. 8192 71.1 / 60.8 and 89.7 /
+// 43.1.)
+__device__ __forceinline__ int adaptive_span(const AttnArgs& a, int L, int step_rows) {
+    const bool seq = int(threadIdx.x & 63) < a.batch;
+    const unsigned steps = seq ? unsigned(max(L, 0) + step_rows - 1) / unsigned(step_rows) : 0u;
+    const unsigned all = __builtin_amdgcn_readlane(wave_inclusive_sum(int(steps)), 63);
+    const unsigned lo = max(1, kMinSpan / step_rows), hi = max(1, a.span_tokens / step_rows);
+    const unsigned target = a.target_splits;
+    unsigned t = target, span;
+    if (!__builtin_amdgcn_ballot_w64(steps * 8 * a.batch > all * 9)) {  // nearly equal
+        const unsigned most = __builtin_amdgcn_readlane(wave_inclusive_max(int(steps)), 63);
+        t = target / a.batch;
+        return int(min(max((most + t - 1) / t, lo), hi));
+    }
+    for (int attempt = 0;; ++attempt) {
+        span = max((all + t - 1) / t, lo);
+        if (attempt == 3) break;
+        const unsigned own = seq ? max(1u, (steps + span - 1) / span) : 0u;
+        const unsigned count = __builtin_amdgcn_readlane(wave_inclusive_sum(int(own)), 63);
+        if (count <= target) break;
+        t = attempt == 2 ? target - a.batch : max(t - min(t, count - target), target - a.batch);
+    }
+    return int(min(span, hi));
 }
 
 // One decode-attention work item: rows [t_begin, t_end) of (sequence b, KV
@@ -877,7 +930,7 @@ __device__ __forceinline__ void decode_attn_seg(const AttnArgs& a, const Seg& sg
     // can reach past the end, where they re-read the split's last step. In
     // paged kernels that round is peeled and loads with the default policy,
     // so the re-reads hit L2 instead of fetching the streamed lines again
-    // (configs[4]-size FP8 batches: 3% less time; batch-1 contiguous launches
+    // (FP8 batches of 128 sequences: 3% less time; batch-1 contiguous launches
     // measured 1% slower with it and keep one loop).
     constexpr int kPeel = PAGED ? 1 : 0;
     AF_STAMP(2);
@@ -1205,6 +1258,7 @@ __device__ __forceinline__ void decode_attn_body(const AttnArgs& a) {
     }
     int hw, split, b;
     int Lc = 0;  // compact grid: the length sequence b attends, from the mapping
+    int span_steps = max(1, a.span_tokens / STEP);
     if (PAGED && a.compact) {
         // Sequence bb owns nhw * splits(L_bb) consecutive workgroup ids.
         auto length = [&](int bb) {
@@ -1226,7 +1280,8 @@ __device__ __forceinline__ void decode_attn_body(const AttnArgs& a) {
             // wave-wide scan and a ballot; no LDS round trip, no barrier).
             const int lane = tid & 63;
             const int Lb = lane < a.batch ? length(lane) : 0;
-            const int n = lane < a.batch ? grid_splits(a, Lb, STEP) : 0;
+            if (a.target_splits > 0) span_steps = adaptive_span(a, Lb, STEP);
+            const int n = lane < a.batch ? grid_splits(a, Lb, STEP, span_steps) : 0;
             const int incl = wave_inclusive_sum(n);
             if (id >= int64_t(__builtin_amdgcn_readlane(incl, 63)) * nhw) return;
             // the first sequence whose splits end past id
@@ -1240,7 +1295,7 @@ __device__ __forceinline__ void decode_attn_body(const AttnArgs& a) {
             if (tid < a.batch) {
                 const int Lb = length(tid);
                 s_len[tid] = Lb;
-                s_splits[tid] = grid_splits(a, Lb, STEP);
+                s_splits[tid] = grid_splits(a, Lb, STEP, span_steps);
             }
             __syncthreads();
             block_exclusive_scan(s_splits, s_first, a.batch);
@@ -1306,7 +1361,7 @@ __device__ __forceinline__ void decode_attn_body(const AttnArgs& a) {
     const int pre_used = below_prefix ? 0 : a.pre_records;  // prefix records this (b, h) merges
     const int t_lo = below_prefix ? 0 : min(a.row_start, L - 1);
     const int total_steps = (L - t_lo + STEP - 1) / STEP;
-    const int n_active = grid_splits(a, L, STEP);
+    const int n_active = grid_splits(a, L, STEP, span_steps);
     if (split >= n_active) return;
     const int step_begin = int(int64_t(split) * total_steps / n_active);
     const int step_end = int(int64_t(split + 1) * total_steps / n_active);
@@ -1828,10 +1883,14 @@ int default_splits(int max_seq_len, int batch, int n_kv_heads) {
     return default_splits_for(max_seq_len, batch, n_kv_heads, true);
 }
 
+// Most rows of a split whose block-table window fits the LDS copy.
+static int max_span_for_table(int block_size) {
+    return (kMaxTableLds - 2) * block_size - 2 * kStepTokens;
+}
+
 // Smallest split count whose span fits the LDS-staged block table.
 static int min_splits_for_table(int max_seq_len, int block_size) {
-    const int max_span = (kMaxTableLds - 2) * block_size - 2 * kStepTokens;
-    return ceil_div(max_seq_len, max_span);
+    return ceil_div(max_seq_len, max_span_for_table(block_size));
 }
 
 }  // namespace af
@@ -2090,14 +2149,22 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
     const int min_sp = min_splits_for_table(std::max(suffix_max, std::min(prefix.len, max_seq_len)), bs);
     int span = kMinSpan;
     bool persistent_ok = false;  // the default partition of a batch may run persistent
+    bool adaptive_ok = false;    // ... or span-adaptive
     if (num_splits <= 0) {
         num_splits = std::max(default_splits_for(suffix_max, batch, nkv, false), min_sp);
         span = default_span(batch, nkv);
         // (FP8 pools; the fp16 kernel streams faster than its per-item
         // set-up and merge let a persistent workgroup overlap, so fp16 batches
-        // keep the grid form)
+        // keep the grid form. And only from about 4096 rows per CU on, where
+        // the persistent form's start and two-sided partition are paid back; us
+        // on MI355X, grid / persistent: 128 sequences of 8192 .. 16384 rows 631
+        // / 576, 64 of the same 325 / 313, 128 of 512 .. 8192 242 / 236; below,
+        // 96 of 512 .. 8192 183 / 195, 48 of 8192 102 / 121, 64 of 512 .. 8192
+        // 130 / 147, 128 of 128 .. 2048 86 / 100, 96 of 64 .. 1024 51 / 66.)
         persistent_ok = fp8 && span == kBatchSpan && prefix.len == 0 && hd == 128 &&
-                        batch <= kMaxPersistBatch;
+                        batch <= kMaxPersistBatch &&
+                        int64_t(batch) * max_seq_len >= int64_t(4096) * device_compute_units();
+        adaptive_ok = prefix.len == 0 && batch > 1 && batch <= kWave && !persistent_ok;
         if (prefix.len > 0 && span == kBatchSpan) {
             // Batched suffixes behind a shared prefix are short: splits of up to
             // ~256 rows (measured best on MI355X for 64 forks of a 2048-row
@@ -2118,9 +2185,34 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
                                        kMaxSplits - num_splits));
         if (num_splits + pre > kMaxSplits) return AF_ERR_OUT_OF_RANGE;
     }
-    const int rec_stride = num_splits + pre;
+    int rec_stride = num_splits + pre;
     if (!workspace || workspace_bytes < attn_workspace_bytes(batch, n_q_heads, hd, rec_stride))
         return AF_ERR_WORKSPACE;
+    // Small batches: spans that follow the lengths (adaptive_span), about one
+    // workgroup per CU, when a (sequence, workgroup column) pair has two CUs or
+    // more and there are rows to spread (shorter launches gain less than the
+    // span's arithmetic costs, 0.3 us). (Three for four CUs: 8 sequences
+    // of 768 .. 12288 fp16 rows 51.9 us against 49.1.) As many records as the
+    // workspace holds, never fewer than the fixed count needs. (Row sums stay
+    // within 31 bits.)
+    int target_splits = 0;
+    int64_t grid = int64_t(batch) * num_splits * nkv;
+    const int cus = device_compute_units();
+    const int nhw = fp8 && nkv % 2 == 0 ? nkv / 2 : nkv;  // workgroups per (sequence, split)
+    const int64_t rows = int64_t(batch) * max_seq_len;
+    if (adaptive_ok && int64_t(batch) * nhw * 2 <= cus && rows > (fp8 ? 2048 : 8192) &&
+        rows < INT32_MAX / 2) {
+        span = max_span_for_table(bs) / kStepTokens * kStepTokens;  // whole steps
+        target_splits = cus / nhw;
+        int n = std::min({target_splits, kMaxSplits, ceil_div(max_seq_len, kMinSpan)});
+        while (n > num_splits &&
+               workspace_bytes < attn_workspace_bytes(batch, n_q_heads, hd, n))
+            --n;
+        num_splits = rec_stride = std::max(num_splits, n);
+        // (splits of the longest span can be more than the target)
+        grid = int64_t(batch) * std::min(num_splits, ceil_div(max_seq_len, span));
+        grid = nkv * std::max<int64_t>(grid, target_splits);
+    }
     const AttnWorkspace w = attn_workspace_carve(workspace, batch, n_q_heads, rec_stride);
     const size_t esz = fp8 ? 1 : 2;
     const size_t slab = size_t(pool->total_blocks) * bs * nkv * hd * esz;
@@ -2151,6 +2243,7 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
     a.n_kv_heads = nkv;
     a.num_splits = num_splits;
     a.span_tokens = span;
+    a.target_splits = target_splits;
     a.qk_scale = qk_scale_for(hd);
     a.scales = fp8 ? pool->scales + size_t(layer) * 2 * nkv : nullptr;
     a.part_o = w.part_o;
@@ -2162,10 +2255,9 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
     a.batch = batch;
     a.cached_rows = (pool->flags & AF_KV_POOL_SHARED_BLOCKS) ? 1 : 0;
     // (Only batched launches without a shared prefix: the shared-prefix form's
-    // short suffix splits measured slower with the length scan, configs[3]
-    // 55.2 against 51.9 us.)
-    a.compact = span == kBatchSpan && pre == 0 && batch <= kThreads;
-    const int64_t grid = int64_t(batch) * num_splits * nkv;
+    // short suffix splits measured slower with the length scan, 64 forks of
+    // 2048 rows 55.2 against 51.9 us.)
+    a.compact = (span == kBatchSpan || target_splits > 0) && pre == 0 && batch <= kThreads;
     if (grid > INT32_MAX) return AF_ERR_UNSUPPORTED;
     if (pre > 0) {  // the prefix's partials first: records 0 .. pre-1
         PrefixPartialArgs pp{};

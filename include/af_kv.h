@@ -231,8 +231,10 @@ int af_paged_rope_append(void* qkv_out, int batch, const af_kv_pool* pool, int l
  * out: [batch, out_stride] fp16. max_seq_len bounds every d_seq_lens[b] and sizes
  * the split grid. Workspace from af_attention_workspace_size(batch, ...).
  * With num_splits = 0, batches of FP8 pools (batch * n_kv_heads * 2 >= CUs,
- * batch <= 256, head_dim 128) run as one persistent launch whose workgroups
- * claim row ranges from a counter in the workspace (re-armed by the launch). */
+ * batch <= 256, head_dim 128) with batch * max_seq_len >= 4096 rows per CU run
+ * as one persistent launch whose workgroups claim row ranges from a counter in
+ * the workspace (re-armed by the launch); small batches take splits whose spans
+ * follow the sequence lengths, as many as the workspace holds records for. */
 int af_paged_attention(const void* q, int q_stride, const af_kv_pool* pool, int layer,
                        const int32_t* d_block_tables, int max_blocks_per_seq,
                        const int32_t* d_seq_lens, int batch, int max_seq_len, void* out,

@@ -409,3 +409,69 @@ def test_paged_fp8_gqa_shapes(gpu, nq, nkv):
         assert np.array_equal(o1.download(np.uint16), o2.download(np.uint16)), layer
     assert np.array_equal(q1.download(np.uint16), q2.download(np.uint16))
     assert np.array_equal(bufs[0].download(np.uint8), bufs[1].download(np.uint8))
+
+
+_SPAN_LENGTHS = {  # lengths of a small batch whose spans follow them
+    "one_long": lambda B, L: [L] + [(0, 1, 31, 64, 65)[b % 5] for b in range(B - 1)],
+    "ragged": lambda B, L: [L] + [int(n) for n in rng(B).integers(1, L + 1, B - 1)],
+    "even": lambda B, L: [L - b for b in range(B)],
+    "tiny": lambda B, L: [1 + b % 3 for b in range(B)],
+}
+
+
+@pytest.mark.parametrize("fp8,B,L", [(False, 2, 4097), (False, 2, 4096), (False, 16, 1025),
+                                     (False, 17, 1025), (True, 2, 4097), (True, 32, 300),
+                                     (True, 33, 300)])
+@pytest.mark.parametrize("kind", sorted(_SPAN_LENGTHS))
+def test_paged_small_batch_spans(gpu, fp8, B, L, kind):
+    """Default splits of small batches, each side of the rule's edges, in a workspace of full and
+    of least size, against the oracle; a replay on other lengths equals the eager launch."""
+    say(f"small batch spans fp8={fp8} B={B} L={L} {kind}")
+    bs = 8 if B == 2 else 16
+    lengths = _SPAN_LENGTHS[kind](B, L)
+    total = sum((L + bs - 1) // bs for _ in lengths) + 3
+    bm = kv.BlockManager(total, bs, 1, dtype=AF_KV_FP8_E4M3 if fp8 else AF_KV_FP16)
+    ids = [bm.allocate_block() for _ in range(total)]
+    for b in rng(771).permutation(ids):
+        bm.free_block(int(b))
+    seqs = _sequences(bm, [L] * B)
+    P = Pool(1, total, bs, fp8, 772)
+    max_blocks = (L + bs - 1) // bs
+    tables, _ = bm.export_tables(seqs, max_blocks)
+    q = randn_f16((B, Q_DIM), 773)
+    d_q, d_t = up(q), up(tables)
+    d_l, d_o = dev.DeviceBuffer(B * 4), dev.DeviceBuffer(B * Q_DIM * 2)
+    least = kv.default_splits(L, B, NKV)
+    stream = dev.Stream()
+    for splits in (0, least):
+        ws = kv.AttentionWorkspace(B, NQ, NKV, HD, splits)
+
+        def launch():
+            kv.launch_paged_attention(d_q, Q_DIM, P.desc, 0, d_t, max_blocks, d_l, B, L, d_o, Q_DIM,
+                                      NQ, ws, stream=stream)
+
+        d_l.upload(np.full(B, L, np.int32))
+        launch()
+        stream.sync()
+        g = dev.Graph.capture(stream, launch)  # captured with other lengths than it replays
+        d_l.upload(np.array(lengths, np.int32))
+        launch()
+        stream.sync()
+        got = d_o.download(np.float16, (B, Q_DIM)).copy()
+        for b in sorted({0, 1, B // 2, B - 2, B - 1}):
+            if lengths[b] == 0:
+                assert not np.any(got[b].view(np.uint16)), b
+                continue
+            args = (q[b], P.slab(0, 0), P.slab(0, 1))
+            tail = (tables[b], lengths[b], bs, NQ, NKV, HD)
+            ref = (oracle.paged_attention_fp8(*args, P.scales[0, 0], P.scales[0, 1], *tail) if fp8
+                   else oracle.paged_attention_f16(*args, *tail))
+            assert_attn_close(got[b], ref, what=f"splits {splits} seq {b} L={lengths[b]}")
+        for _ in range(3):
+            d_o.upload(np.zeros(B * Q_DIM, np.float16))
+            g.launch(stream)
+            stream.sync()
+            assert np.array_equal(d_o.download(np.float16, (B, Q_DIM)).view(np.uint16),
+                                  got.view(np.uint16))
+        g.destroy()
+    bm.close()

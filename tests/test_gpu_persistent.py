@@ -167,3 +167,58 @@ def test_persistent_graph_replays(gpu):
     finally:
         g.destroy()
     bm.close()
+
+
+@pytest.mark.parametrize("below", [False, True])
+def test_persistent_bound_vs_oracle(gpu, below):
+    """Either side of the persistent form's row rule: batch * max_seq_len rows, 4096 per CU.
+
+    The bound, not the lengths, chooses the form, so short sequences reach both; fused and
+    unfused launches agree bit for bit, and so do replays of the captured unfused launch.
+    """
+    B = 96
+    lengths = [min(n, 1500) for n in _lengths(960, B)]
+    lengths[0] = 5  # fused decode appends to every sequence
+    bound = -(-4096 * dev.device_info()["compute_units"] // B) - int(below)
+    say(f"persistent bound B={B} bound={bound}")
+    bm, seqs, P = _batch(lengths, 961)
+    bs = P.bs
+    slots, positions, copies = bm.plan_decode(seqs)
+    max_blocks = (bound + bs - 1) // bs
+    tables, lens = bm.export_tables(seqs, max_blocks)
+    max_pos = max(lengths) + 2
+    c, s = oracle.rope_table(max_pos, HD, THETA)
+    d_c, d_s = up(c), up(s)
+    d_qkv, d_t, d_l = up(randn_f16((B, QKV), 962)), up(tables), up(lens)
+    d_sl, d_p = up(slots), up(positions)
+    d_o1, d_o2 = dev.DeviceBuffer(B * Q_DIM * 2), dev.DeviceBuffer(B * Q_DIM * 2)
+    ws = kv.AttentionWorkspace(B, NQ, NKV, HD, 0)
+    stream = dev.Stream()
+    kv.launch_paged_decode_fused(d_qkv, B, P.desc, 1, d_sl, d_p, d_c, d_s, max_pos, d_t,
+                                 max_blocks, bound, d_o1, Q_DIM, NQ, ws, stream=stream)
+
+    def launch():
+        kv.launch_paged_attention(d_qkv, QKV, P.desc, 1, d_t, max_blocks, d_l, B, bound, d_o2,
+                                  Q_DIM, NQ, ws, stream=stream)
+
+    launch()
+    stream.sync()
+    got = d_o2.download(np.float16, (B, Q_DIM)).copy()
+    assert np.array_equal(bits(d_o1.download(np.float16, (B, Q_DIM))), bits(got))
+    q, pool = d_qkv.download(np.float16, (B, QKV))[:, :Q_DIM], P.download()
+    for b in list(range(6)) + list(range(20, B, 15)):
+        ref = oracle.paged_attention_fp8(q[b], pool[1, 0], pool[1, 1], P.scales[1, 0],
+                                         P.scales[1, 1], tables[b], lengths[b] + 1, bs, NQ, NKV, HD)
+        assert_attn_close(got[b], ref, what=f"seq {b}")
+    g = dev.Graph.capture(stream, launch)
+    try:
+        for i in range(3):
+            d_o2.upload(np.zeros(B * Q_DIM, np.float16))
+            g.launch(stream)
+            stream.sync()
+            assert np.array_equal(bits(d_o2.download(np.float16, (B, Q_DIM))), bits(got)), i
+            launch()
+            stream.sync()
+    finally:
+        g.destroy()
+    bm.close()
