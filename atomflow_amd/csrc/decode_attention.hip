@@ -158,10 +158,6 @@ struct AttnArgs {
     int32_t n_kv_heads;
     int32_t num_splits;
     int32_t span_tokens;  // target tokens per split: a sequence uses ceil(L / span) splits
-    // Compact grid of up to 64 sequences, target_splits > 0: every sequence's span
-    // is the smallest (at least kMinSpan, at most span_tokens) with which the
-    // batch has at most target_splits splits (see adaptive_span).
-    int32_t target_splits;
     float qk_scale;       // log2(e) / sqrt(head_dim)
     const float* scales;  // FP8: [2][n_kv_heads] (K, V) of this layer
     float* part_o;        // [batch][n_kv_heads][rec_stride][GROUP * head_dim]
@@ -193,6 +189,10 @@ struct AttnArgs {
     // the CACHED kernels, which read KV rows with the ordinary cache policy
     // instead of non-temporal loads.
     int32_t cached_rows;
+    // Compact grid of up to 64 sequences, target_splits > 0: every sequence's span
+    // is the smallest (at least kMinSpan, at most span_tokens) with which the
+    // batch has at most target_splits splits (see adaptive_span).
+    int32_t target_splits;
 };
 
 template <int HD, bool FP8>
