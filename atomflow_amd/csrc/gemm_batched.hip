@@ -11,6 +11,10 @@
 // and writes K and V to each token's slot of the paged pool, exactly as
 // af_paged_rope_append does on the projection's output.
 //
+// Every kernel here sums a token's products in one order (a fresh fragment per
+// quantisation group, the groups of each of eight parts of K, the parts), so a
+// token's result has the same bits whatever launch it is in, from two tokens on.
+//
 // Few tokens (w8a16_batched_kernel; HBM-bound: one weight byte per 2*M flops, M
 // <= 32 per workgroup). Launches of more tokens or rows take the tiled kernel
 // further down (pick_tile):
@@ -33,6 +37,7 @@
 //    RoPE runs on the rounded fp16 projections.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "af_common.h"
 #include "af_device.h"
@@ -327,11 +332,8 @@ __global__ __launch_bounds__(kBgThreads, 4) void w8a16_batched_kernel(const Batc
 // little arithmetic: each workgroup re-reads the activations of its tokens (the
 // 16-row kernel above reads all of x per 16 rows and the weights once per 32
 // tokens), and the matrix cores have work. The tiled kernel gives a workgroup BM
-// tokens x BN weight rows and, with KS > 1, KS group-aligned parts of K; a wave
-// owns a (BM / WR) x (BN / WC) piece of one part as 32x32x16 MFMAs. 2011 tokens
-// of 8192 x 3072: 470 us on the 16-row kernel, 108 here (0.95 PFLOP/s); a bare
-// loop of the same MFMAs and barriers takes 77, the DMA, the operand reads and
-// the group scales about 10 each; 64 tokens of 3072 x 8192: 25.7 and 16.6 us.
+// tokens x BN weight rows; its KS groups of waves take 8 / KS of the eight parts of
+// K each, and a wave owns a (BM / WR) x (BN / WC) piece as 32x32x16 MFMAs.
 //  * K advances 64 per step. A step's x rows (128 B each, fp16) and weight rows
 //    (64 B each, E4M3) go from global memory straight into LDS (lds_dma16), in a
 //    ring of ST stages: the loads of step s + ST - 1 are issued in step s, one
@@ -340,24 +342,30 @@ __global__ __launch_bounds__(kBgThreads, 4) void w8a16_batched_kernel(const Batc
 //  * 16-byte chunks are XOR-swizzled (x by row / 2, weights by row / 4) so that
 //    an operand read of 16 rows covers every bank once; the swizzle is made by
 //    choosing which chunk each DMA lane fetches.
-//  * A lane reads 16 weight bytes for two MFMAs: of 32 k, lanes 0-31 hold the
-//    first 16 and lanes 32-63 the last; x is read in the same k order.
-//  * Group scales: D's column is the lane's weight row, so a group's scale is
-//    one value per lane and column tile. The accumulator is kept in units of
-//    the current group's scale: entering group g it is multiplied by
-//    scale[g-1] / scale[g] (one multiply per element and group), at the end by
-//    the last scale. (A second accumulator per group, added with its scale,
-//    would double the accumulator registers.) A zero scale counts as 2^-66,
-//    whose group then adds less than half the smallest fp16. Scales are staged
-//    in LDS eight groups at a time: a register load waited for in each group
-//    would drain the DMA ring with it.
-//  * The parts of K are summed through LDS in a fixed order, and the tile leaves
+//  * The sums are the 16-row kernel's, bit for bit. There, a 16x16x32 MFMA takes
+//    bytes 8v .. 8v+7 of each 16 of a 64-k chunk, v = 0 then 1; the hardware adds a
+//    16x16x32 product's two halves of K one after the other, exactly as two 32x32x16
+//    MFMAs do (compared on random, subnormal, infinite and NaN operands), so a step
+//    runs v over both halves of the chunk before the next v. A group's products
+//    start from zero, then acc = fma(scale, products, acc), so zero and non-finite
+//    scales and activations act as they do there. Parts are added in order, part 0
+//    first.
+//  * That takes three accumulators per output where K is not cut over waves (group,
+//    part, total), and the register file then holds two waves of 64 x 64 per SIMD:
+//    2011 tokens of 8192 x 3072 take 109 us (0.93 PFLOP/s; 16-row kernel 432, one
+//    rescaled accumulator with four waves per SIMD 101, but its bits depended on the
+//    tile), 3072 x 8192 121 (509, 137); 64 tokens of 3072 x 8192 17.2 (26.2, 17.6).
+//    With two waves the MFMAs of one run beside the conversions and the fold of the
+//    other only in part; issue priority for the wave in its MFMAs is worth 3-5 %.
+//  * Group scales: D's column is the lane's weight row, so a group's scale is one
+//    value per lane and column tile. Scales are staged in LDS eight groups at a time:
+//    a register load waited for in each group would drain the DMA ring with it.
+//  * Parts of K on different waves are summed through LDS, and the tile leaves
 //    through LDS as fp16, so rows are stored 16 B per lane. In the fused kernel
 //    the BN columns are BN / 2 dims d of a head and their partners d + 64, and
 //    each thread rotates and appends 8 such pairs of a token from there.
 //  * Workgroups are dealt so that each XCD owns whole column panels (its L2
 //    then reads each weight once and x once).
-constexpr float kZeroScale = 0x1p-66f;
 constexpr int kScaleChunk = 8;  // groups staged at a time
 
 template <int BM, int BN, int KS, int ST>
@@ -368,8 +376,11 @@ struct TileLayout {
     static constexpr int kStage = KS * kPart;
     static constexpr int kRing = ST * kStage;
     static constexpr int kOutStride = BN * 2 + 16;  // bytes between output rows in LDS
-    static constexpr int kRed = KS > 1 ? KS * BM * BN * 4 : 0;
-    static constexpr int kTail = kRed + BM * kOutStride;
+    static constexpr int kParts = kBgParts / KS;  // parts of K per wave
+    // Sums left for the others: one of the first waves' parts, then each part's.
+    static constexpr int kSlots = KS > 1 ? 1 + (KS - 1) * kParts : 0;
+    static constexpr int kRed = kSlots * BM * BN * 4;
+    static constexpr int kTail = kRed > BM * kOutStride ? kRed : BM * kOutStride;
     static constexpr int kScales = kRing;  // [2][KS][kScaleChunk][BN] fp16 after the ring
     static constexpr int kScaleBytes = ST > 2 ? 2 * KS * kScaleChunk * BN * 2 : 0;
     static constexpr int kLds =
@@ -496,6 +507,7 @@ w8a16_tiled_kernel(const BatchedArgs a) {
     // register load of the next group's scales costs no wait of its own.
     constexpr bool kRegScales = ST == 2;
     static_assert(ST >= 2, "a stage is read while the next one loads");
+    static_assert(KS == 1 || kBgParts <= 2 * KS, "a wave keeps at most two parts' sums apart");
     static_assert(MT >= 1 && NT >= 1 && XI >= 1 && WI >= 1, "tile too small for its waves");
     static_assert(XI * 8 * NW == BM && WI * 16 * NW == BN && BN <= 64 * NW, "uneven DMA");
     __shared__ __align__(16) char s_lds[L::kLds];
@@ -513,11 +525,13 @@ w8a16_tiled_kernel(const BatchedArgs a) {
     const int tile = xcd * per + min(xcd, rest) + (int(blockIdx.x) >> 3);
     const int t0 = (tile % mb) * BM, pn = tile / mb;
 
-    // This wave's part of K, in groups and 64-k steps.
-    const int g_lo = ks * a.groups / KS, g_hi = (ks + 1) * a.groups / KS;
+    // This wave's parts of K, in groups and 64-k steps.
+    constexpr int kParts = L::kParts;
+    auto part_begin = [&](int p) { return p * a.groups / kBgParts; };
+    const int g_lo = part_begin(ks * kParts), g_hi = part_begin((ks + 1) * kParts);
     const int per_group = a.group_size / 64;
     const int steps = (g_hi - g_lo) * per_group;
-    const int all_steps = (a.groups + KS - 1) / KS * per_group;  // the longest part's
+    const int all_steps = (a.groups + KS - 1) / KS * per_group;  // the longest wave's
 
     // DMA sources: one scalar base per operand, 32-bit lane offsets. Rows past m
     // or n load the last row: their products are not stored.
@@ -594,17 +608,19 @@ w8a16_tiled_kernel(const BatchedArgs a) {
         wa[p] = ks * L::kPart + L::kXBytes + uint32_t(wr) * 64u +
                 16u * uint32_t((2 * p + hi) ^ ((wr >> 2) & 3));
 
-    float16v_t acc[MT][NT];
-    float scale[NT];
+    // f: the current group's products; acc: the current part's sum; done: the sum of
+    // the wave's parts before it (one part per wave: unused).
+    float16v_t f[MT][NT], acc[MT][NT], done[MT][NT];
+    float scale[NT];  // the current group's
+    float16v_t zero;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) zero[r] = 0.0f;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        scale[nt] = 1.0f;
+        scale[nt] = 0.0f;
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
+        for (int mt = 0; mt < MT; ++mt) f[mt][nt] = acc[mt][nt] = done[mt][nt] = zero;
     }
-
     uint16_t sraw[NT];  // kRegScales: the next group's scales
     const uint16_t* slane[NT];
 #pragma unroll
@@ -613,61 +629,60 @@ w8a16_tiled_kernel(const BatchedArgs a) {
                     size_t(min(panel_row<FUSED, BN>(pn, wr + 32 * nt), a.n - 1)) * a.groups;
         if constexpr (kRegScales) sraw[nt] = slane[nt][min(g_lo, a.groups - 1)];
     }
-    int left = 0;    // steps of the current group still to come
-    int group = -1;  // the current group of the part
-    int buf = 0;
-    for (int st = 0; st < all_steps; ++st) {
-        // This step's loads have arrived (the D - 1 later steps' may be in
-        // flight); the barrier covers the other waves' and frees the buffer read
-        // a step ago.
+    // Adds the finished group's products to the part's sum.
+    auto fold = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    acc[mt][nt][r] = fmaf(scale[nt], f[mt][nt][r], acc[mt][nt][r]);
+    };
+    auto end_part = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    done[mt][nt][r] += acc[mt][nt][r];
+                    acc[mt][nt][r] = 0.0f;
+                }
+    };
+    using No = std::integral_constant<bool, false>;
+    using Yes = std::integral_constant<bool, true>;
+    int st = 0, buf = 0;
+    // Before step st: its loads have arrived (the D - 1 later steps' may be in
+    // flight); the barrier covers the other waves' and frees the buffer read a step
+    // ago, which step st + D's loads go to.
+    auto arrive = [&]() __attribute__((always_inline)) {
         if (st + D - 1 < steps) wait_vmcnt<(D - 1) * (XI + WI)>();
         else wait_vmcnt<0>();
         __syncthreads();
-        if (KS > 1 && st >= steps) continue;  // a shorter part waits for the others
-        if (left == 0) {  // a group begins: the accumulator moves to its scale
-            left = per_group;
-            ++group;
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                float v;
-                if constexpr (kRegScales)
-                    v = h2f(sraw[nt]);
-                else
-                    v = h2f(s_scale[((((group / kScaleChunk) & 1) * KS + ks) * kScaleChunk +
-                                     group % kScaleChunk) * BN + wr + 32 * nt]);
-                const float sc = v == 0.0f ? kZeroScale : v;
-                if (group > 0) {
-                    const float ratio = scale[nt] / sc;
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[mt][nt][r] *= ratio;
-                }
-                scale[nt] = sc;
-                if constexpr (kRegScales)
-                    sraw[nt] = slane[nt][min(g_lo + group + 1, a.groups - 1)];
-            }
-            if constexpr (!kRegScales)
-                if (group % kScaleChunk == kScaleChunk - 1) {  // read a group later
-                    const int c = group / kScaleChunk + 1;
-                    stage_scales(c);
-                    load_scales(c + 1);
-                }
-        }
-        --left;
+    };
+    auto ahead = [&]() __attribute__((always_inline)) {
         if (st + D < steps) issue(st + D, buf == 0 ? D : buf - 1);
+    };
+    // One 64-k step; FIRST of a group: the products start from zero.
+    auto products = [&](auto first_c) __attribute__((always_inline)) {
+        if constexpr (KS == 1) __builtin_amdgcn_s_setprio(1);
         const char* s = s_lds + buf * L::kStage;
+        uint4 wv[2][NT];
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            half8_t wf[NT][2];
+        for (int p = 0; p < 2; ++p)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const uint4 v = *reinterpret_cast<const uint4*>(s + wa[p] + nt * 32 * 64);
-                wf[nt][0] = e4m3x8(v.x, v.y);
-                wf[nt][1] = e4m3x8(v.z, v.w);
-            }
+            for (int nt = 0; nt < NT; ++nt)
+                wv[p][nt] = *reinterpret_cast<const uint4*>(s + wa[p] + nt * 32 * 64);
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                half8_t wf[NT];
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+                    wf[nt] = j == 0 ? e4m3x8(wv[p][nt].x, wv[p][nt].y)
+                                    : e4m3x8(wv[p][nt].z, wv[p][nt].w);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     const half8_t xf = __builtin_bit_cast(
@@ -675,20 +690,60 @@ w8a16_tiled_kernel(const BatchedArgs a) {
                         *reinterpret_cast<const uint4*>(s + xa[2 * p + j] + mt * 32 * 128));
 #pragma unroll
                     for (int nt = 0; nt < NT; ++nt)
-                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf, wf[nt][j],
-                                                                             acc[mt][nt], 0, 0, 0);
+                        f[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            xf, wf[nt], decltype(first_c)::value && j + p == 0 ? zero : f[mt][nt], 0,
+                            0, 0);
                 }
-        }
+            }
+        if constexpr (KS == 1) __builtin_amdgcn_s_setprio(0);
+        ++st;
         buf = buf == D ? 0 : buf + 1;
+    };
+    int part = ks * kParts;               // the current part
+    int part_end = part_begin(part + 1);  // its last group + 1
+    for (int group = g_lo; group < g_hi; ++group) {
+        arrive();
+        const int gl = group - g_lo;
+        if constexpr (!kRegScales)
+            if (gl % kScaleChunk == kScaleChunk - 1) {  // read a group later
+                const int c = gl / kScaleChunk + 1;
+                stage_scales(c);
+                load_scales(c + 1);
+            }
+        ahead();
+        fold();
+        if (kParts > 1 && group == part_end) {
+            end_part();
+            do part_end = part_begin(++part + 1);
+            while (part_end <= group);
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            if constexpr (kRegScales) {
+                scale[nt] = h2f(sraw[nt]);
+                sraw[nt] = slane[nt][min(group + 1, a.groups - 1)];
+            } else {
+                scale[nt] = h2f(s_scale[((((gl / kScaleChunk) & 1) * KS + ks) * kScaleChunk +
+                                         gl % kScaleChunk) * BN + wr + 32 * nt]);
+            }
+        }
+        products(Yes{});
+        for (int i = 1; i < per_group; ++i) {
+            arrive();
+            ahead();
+            products(No{});
+        }
     }
+    for (; st < all_steps; ++st) arrive();  // a wave of fewer steps keeps the others' barriers
+    fold();
+    if constexpr (KS == 1) end_part();
 
     // Register r of (mt, nt) is token 32 mt + 8 (r / 4) + 4 hi + r % 4 of the
     // wave's piece, column 32 nt + col.
     __syncthreads();
-    char* s_out = s_lds + L::kRed;
     auto put = [&](int mt, int nt, int r, float v) {
         const int row = wm + 32 * mt + 8 * (r >> 2) + 4 * hi + (r & 3);
-        *reinterpret_cast<uint16_t*>(s_out + row * L::kOutStride + 2 * (wr + 32 * nt)) = f2h(v);
+        *reinterpret_cast<uint16_t*>(s_lds + row * L::kOutStride + 2 * (wr + 32 * nt)) = f2h(v);
     };
     if constexpr (KS == 1) {
 #pragma unroll
@@ -696,40 +751,57 @@ w8a16_tiled_kernel(const BatchedArgs a) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) put(mt, nt, r, acc[mt][nt][r] * scale[nt]);
+                for (int r = 0; r < 16; ++r) put(mt, nt, r, done[mt][nt][r]);
     } else {
-        // Every part leaves its sums in LDS; each part's waves add a 16 / KS
-        // share of the registers over the parts, part 0 first.
+        // The waves of the first parts leave their total in LDS, the others each
+        // part's sum; each wave adds up a 16 / KS share of the registers.
         float* red = reinterpret_cast<float*>(s_lds);
-        auto at = [&](int part, int mt, int nt, int r) {
-            return ((((part * NW + wave) * MT + mt) * NT + nt) * 16 + r) * 64 + lane;
+        auto at = [&](int slot, int mt, int nt, int r) {
+            return ((((slot * NW + wave) * MT + mt) * NT + nt) * 16 + r) * 64 + lane;
         };
+        constexpr int RS = 16 / KS;
+        float v[MT][NT][RS];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) red[at(ks, mt, nt, r)] = acc[mt][nt][r] * scale[nt];
+                for (int r = 0; r < 16; ++r) {
+                    // (slot 0: the first wave's parts; then part kParts, ..)
+                    const int slot = ks == 0 ? 0 : 1 + (ks - 1) * kParts;
+                    const float d = done[mt][nt][r], s = acc[mt][nt][r];
+                    if (kParts == 1 || ks == 0) {
+                        red[at(slot, mt, nt, r)] = kParts == 1 ? s : d + s;
+                    } else {
+                        red[at(slot, mt, nt, r)] = d;
+                        red[at(slot + 1, mt, nt, r)] = s;
+                    }
+                }
         __syncthreads();
-        constexpr int RS = 16 / KS;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                 for (int i = 0; i < RS; ++i) {
-                    const int r = ks * RS + i;
-                    float v = red[at(0, mt, nt, r)];
+                    v[mt][nt][i] = red[at(0, mt, nt, ks * RS + i)];
 #pragma unroll
-                    for (int part = 1; part < KS; ++part) v += red[at(part, mt, nt, r)];
-                    put(mt, nt, r, v);
+                    for (int q = 1; q < L::kSlots; ++q)
+                        v[mt][nt][i] += red[at(q, mt, nt, ks * RS + i)];
                 }
+        __syncthreads();
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int i = 0; i < RS; ++i) put(mt, nt, ks * RS + i, v[mt][nt][i]);
     }
     __syncthreads();
     if constexpr (FUSED)
-        store_tile_rope<FP8, BM, BN, THREADS, L::kOutStride>(a, s_out, t0, pn, tid);
+        store_tile_rope<FP8, BM, BN, THREADS, L::kOutStride>(a, s_lds, t0, pn, tid);
     else
-        store_tile<BM, BN, THREADS, L::kOutStride>(a, s_out, t0, pn * BN, tid);
+        store_tile<BM, BN, THREADS, L::kOutStride>(a, s_lds, t0, pn * BN, tid);
 }
 
 template <bool FUSED, bool FP8, int BM, int BN, int WR, int WC, int KS, int ST, int WGS>
@@ -739,40 +811,43 @@ void launch_tiled(const BatchedArgs& a, hipStream_t s) {
                        dim3(64 * WR * WC * KS), 0, s, a);
 }
 
-// The tiles, and what a launch of each was measured to cost on MI355X (nine
-// (n, k) shapes from 2048 x 8192 to 14336 x 4096, 16 to 4000 tokens; the model
-// below fits each within 5-9 % rms): a round of workgroups, `wgs` of them per CU
-// while tiles last, takes `round` plus per 64-k step `step` and, for each
-// workgroup that shares the CU, `share` (us); a launch `fixed` besides. Small
-// tiles with several parts of K fill the device when tokens or rows are few
-// (their weights and x are then read by more workgroups), large ones read the
-// least and keep the matrix cores busiest.
+// The forms, and what a launch of each was measured to cost on MI355X (eleven
+// (n, k) shapes from 4100 x 640 to 14336 x 4096, 2 to 4096 tokens; the model below
+// fits each within 3-9 % rms where it is near the best): a round of workgroups,
+// `wgs` of them per CU while tiles last, takes `round` plus per 64-k step `step`,
+// for each workgroup of the busiest CUs `share` and for each workgroup of the average
+// CU `spread` (us); a launch `fixed` besides. Small tiles with several parts of K at a
+// time fill the device when tokens or rows are few (their weights and x are then read
+// by more workgroups), large ones read the least and keep the matrix cores busiest.
 struct TileCost {
     int bm, bn, ks, wgs;
-    float fixed, step, share, round;
+    float fixed, round, step, share, spread;
 };
-enum { kT128x256, kT128x128, kT64x128, kT64x64k2, kT128x64k2, kT64x64k4, kT64x32k4, kT32x32k4,
-       kT32x32k8, kTiles };
+enum { kT128x128, kT64x128, kT64x64, kT64x64k4, kT64x32k4, kT32x64k4, kT32x32k8, kRows16, kRows32,
+       kTiles };
 constexpr TileCost kTileCost[kTiles] = {
-    {128, 256, 1, 2, 0.0f, 0.0f, 0.940f, 5.94f},      {128, 128, 1, 3, 0.0f, 0.234f, 0.447f, 3.20f},
-    {64, 128, 1, 4, 0.0f, 0.346f, 0.185f, 1.57f},     {64, 64, 2, 2, 0.83f, 0.180f, 0.312f, 2.65f},
-    {128, 64, 2, 1, 0.0f, 0.698f, 0.0f, 4.33f},       {64, 64, 4, 1, 0.0f, 0.923f, 0.0f, 3.13f},
-    {64, 32, 4, 1, 0.71f, 0.582f, 0.0f, 2.59f},       {32, 32, 4, 2, 2.11f, 0.161f, 0.282f, 1.30f},
-    {32, 32, 8, 1, 1.41f, 0.759f, 0.0f, 2.60f}};
+    {128, 128, 1, 2, 1.495f, 10.360f, 0.237f, 0.142f, 0.243f},
+    {64, 128, 1, 3, 0.0f, 7.508f, 0.275f, 0.0f, 0.219f},
+    {64, 64, 1, 3, 2.463f, 3.766f, 0.148f, 0.048f, 0.089f},
+    {64, 64, 4, 1, 3.304f, 2.710f, 0.660f, 0.0f, 0.252f},
+    {64, 32, 4, 1, 2.402f, 2.503f, 0.467f, 0.0f, 0.113f},
+    {32, 64, 4, 1, 3.203f, 1.723f, 0.477f, 0.0f, 0.159f},
+    {32, 32, 8, 1, 3.410f, 1.087f, 0.584f, 0.0f, 0.296f},
+    // the 16-row kernel, up to 16 tokens and from 17 on
+    {16, 16, 8, 2, 2.584f, 0.0f, 0.156f, 0.403f, 0.203f},
+    {32, 16, 8, 4, 3.000f, 0.0f, 0.147f, 0.428f, 0.285f}};
 
-// The cheapest tile by kTileCost, or -1 for the 16-row kernel above: group sizes
-// that are not whole 64-k steps, strides past the 32-bit lane offsets, and
-// launches of at most one 16-row workgroup per CU, whose eight K parts then
-// stream the weights faster than any tile (3072 rows of k 3072: 16 tokens 6.1 us
-// against 7.0, 32 tokens 7.0 against 7.8; at 48 tokens, past one workgroup per
-// CU, 10.3 against 7.9). The choice depends on (m, n, k, group size) alone, so
-// the fused kernel and the plain projection always sum in the same order.
+// The cheapest form by kTileCost; kRows16 also for what the tiles do not take: group
+// sizes that are not whole 64-k steps and strides past the 32-bit lane offsets. Of the
+// measured launches it picks one within 1.3 % of the best on average (17 % at most).
+// (us, 16-row kernel / best tile: 3072 rows of k 8192, 16 tokens 14.0 / 15.9, 33 tokens
+// 26 / 16.5; 4100 rows of k 640, 16 tokens 4.4 / 5.2; 5120 rows of k 3072, 2 tokens
+// 9.9 / 8.6.) All forms give the same bits.
 int pick_tile(const BatchedArgs& a) {
     if (a.group_size % 64 != 0 || a.x_stride >= (int64_t(1) << 23) || a.k >= (1 << 24) ||
         int64_t(a.m) * a.n >= (int64_t(1) << 40))
-        return -1;
+        return kRows16;
     const unsigned cus = unsigned(device_compute_units());
-    if (int64_t(ceil_div(a.n, kBgRows)) * ceil_div(a.m, 2 * kBgTile) <= int64_t(cus)) return -1;
     // (called for every launch: constant tile sizes, 32-bit arithmetic)
     const unsigned m = unsigned(a.m), n = unsigned(a.n), groups = unsigned(a.groups);
     const float per_group = float(a.group_size / 64);
@@ -781,13 +856,14 @@ int pick_tile(const BatchedArgs& a) {
 #pragma clang loop unroll(full)
     for (int i = 0; i < kTiles; ++i) {
         constexpr auto up = [](unsigned x, int by) { return (x + by - 1) / unsigned(by); };
+        if (i == (a.m > kBgTile ? kRows16 : kRows32)) continue;
         const TileCost& c = kTileCost[i];
-        const unsigned tiles = up(m, c.bm) * up(n, c.bn);  // (m n < 2^40 over 32 x 32 at least)
+        const unsigned tiles = up(m, c.bm) * up(n, c.bn);  // (m n < 2^40 over 32 x 16 at least)
         const unsigned per_cu = (tiles + cus - 1) / cus;   // shares of the launch's busiest CUs
         const unsigned rounds = up(per_cu, c.wgs);
         const float steps = float(up(groups, c.ks)) * per_group;
         const float cost = c.fixed + float(rounds) * (c.round + steps * c.step) +
-                           float(per_cu) * steps * c.share;
+                           steps * (float(per_cu) * c.share + float(tiles) / float(cus) * c.spread);
         if (i == 0 || cost < best_cost) {
             best = i;
             best_cost = cost;
@@ -799,17 +875,12 @@ int pick_tile(const BatchedArgs& a) {
 template <bool FUSED, bool FP8>
 void launch_tile(int tile, const BatchedArgs& a, hipStream_t s) {
     switch (tile) {
-        case kT128x256:
-            // (a fused panel is at most one head; the same sums in 128 columns)
-            if constexpr (!FUSED) return launch_tiled<FUSED, FP8, 128, 256, 2, 4, 1, 2, 2>(a, s);
-            [[fallthrough]];
-        case kT128x128: return launch_tiled<FUSED, FP8, 128, 128, 1, 4, 1, 2, 3>(a, s);
-        case kT64x128: return launch_tiled<FUSED, FP8, 64, 128, 1, 4, 1, 2, 4>(a, s);
-        case kT64x64k2: return launch_tiled<FUSED, FP8, 64, 64, 2, 2, 2, 3, 2>(a, s);
-        case kT128x64k2: return launch_tiled<FUSED, FP8, 128, 64, 2, 2, 2, 3, 1>(a, s);
-        case kT64x64k4: return launch_tiled<FUSED, FP8, 64, 64, 2, 1, 4, 3, 1>(a, s);
+        case kT128x128: return launch_tiled<FUSED, FP8, 128, 128, 2, 2, 1, 3, 2>(a, s);
+        case kT64x128: return launch_tiled<FUSED, FP8, 64, 128, 1, 4, 1, 2, 3>(a, s);
+        case kT64x64: return launch_tiled<FUSED, FP8, 64, 64, 2, 2, 1, 3, 4>(a, s);
+        case kT64x64k4: return launch_tiled<FUSED, FP8, 64, 64, 1, 2, 4, 3, 1>(a, s);
         case kT64x32k4: return launch_tiled<FUSED, FP8, 64, 32, 2, 1, 4, 3, 1>(a, s);
-        case kT32x32k4: return launch_tiled<FUSED, FP8, 32, 32, 1, 1, 4, 3, 2>(a, s);
+        case kT32x64k4: return launch_tiled<FUSED, FP8, 32, 64, 1, 2, 4, 3, 1>(a, s);
         default: return launch_tiled<FUSED, FP8, 32, 32, 1, 1, 8, 3, 1>(a, s);
     }
 }
@@ -817,7 +888,7 @@ void launch_tile(int tile, const BatchedArgs& a, hipStream_t s) {
 template <bool FUSED, bool FP8>
 void launch_batched(const BatchedArgs& a, int row_blocks, hipStream_t s) {
     const int tile = pick_tile(a);
-    if (tile >= 0) return launch_tile<FUSED, FP8>(tile, a, s);
+    if (tile < kRows16) return launch_tile<FUSED, FP8>(tile, a, s);
     const bool two = a.m > kBgTile;
     const int per = kBgTile * (two ? 2 : 1);
     const dim3 grid(row_blocks, (a.m + per - 1) / per), block(kBgThreads);

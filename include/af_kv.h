@@ -332,7 +332,9 @@ int af_w8a16_gemv_pair(const void* x, const uint8_t* weight0, const void* scales
  * token per step: launch_w8a16_gemv, qkv_gemm.cu:32-152; a serving step has one
  * token per sequence). k and group_size multiples of 32; x_stride >= k and a
  * multiple of 8; x and weight 16-byte aligned. m = 1 runs af_w8a16_gemv itself
- * (the same bits); more tokens take matrix-core tiles sized by (m, n, k). */
+ * (the same bits); more tokens take matrix-core tiles sized by (m, n, k), which
+ * all sum in one order: for m >= 2 a token's row has the same bits whatever m, n
+ * and the other tokens are (a prompt may be chunked anywhere). */
 int af_w8a16_gemm_batched(const void* x, int64_t x_stride, int m, const uint8_t* weight,
                           const void* scales, void* y, int64_t y_stride, int n, int k,
                           int group_size, af_stream_t stream);

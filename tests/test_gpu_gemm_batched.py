@@ -205,7 +205,7 @@ def deq(w, s, group):
 @pytest.mark.parametrize("n,k,m,group,y_off", [
     (4100, 64, 2, 64, 0), (4100, 640, 33, 128, 1), (4100, 640, 2, 128, 0), (1000, 640, 520, 128, 1),
     (1000, 1024, 520, 128, 0), (4100, 3072, 2, 128, 0), (8200, 1536, 65, 512, 0),
-    (8200, 3072, 65, 128, 0), (4100, 128, 2100, 128, 0), (3072, 3072, 2100, 128, 0)])
+    (8200, 3072, 65, 128, 0), (4100, 128, 2100, 128, 0), (3072, 3072, 2100, 128, 0), (4100, 640, 1000, 128, 1)])
 def test_gemm_tiled_parity(gpu, n, k, m, group, y_off):
     """One case or more for each tile of the tiled kernel, with partial token and
     column tiles, fewer groups than K parts, parts of unequal length, output rows
@@ -274,3 +274,49 @@ def test_paged_qkv_rope_append_many_tokens(gpu, fp8, m, q_off):
     assert np.array_equal(got, want)
     assert np.array_equal(pools[0][0].download(np.uint8), pools[1][0].download(np.uint8))
     assert st.download(np.int32, (1,))[0] == atomflow_amd.AF_ERR_OUT_OF_RANGE
+
+
+def odd_values(w, s, x):
+    """Zero, subnormal, negative, huge, infinite and NaN group scales, infinite and NaN
+    activations in and out of zero-scale groups, and a NaN weight code."""
+    w, s, x = w.copy(), s.copy(), x.copy()
+    s[0, 0] = s[1, -1] = 0.0
+    s[2, :] = 0.0
+    s[3, 0] = s[3, -1] = np.inf
+    s[4, s.shape[1] // 2] = np.nan
+    s[5, 0], s[5, -1] = np.float16(6e-8), 65504.0
+    s[6, :] = -s[6, :]
+    s[7, -1] = -np.inf
+    w[9, 3] = 0x7f
+    x[0, 1], x[1, -1], x[-1, 0] = np.inf, -np.inf, np.nan
+    x[-2, ::2], x[-2, 1::2] = 65504.0, -65504.0
+    return w, s, x
+
+
+# one or more of every form: the 16-row kernel's two, and each tile; group sizes of one to
+# sixteen 64-k steps, from one group to more than eight per part, fewer groups than parts
+@pytest.mark.parametrize("n,k,m,group", [
+    (4100, 640, 20, 128), (5125, 3072, 5, 128), (3072, 8192, 17, 128), (5125, 3072, 33, 128),
+    (4100, 4608, 40, 192), (5125, 3072, 70, 128), (4100, 1536, 70, 512), (5125, 3072, 129, 128),
+    (1000, 1024, 517, 128), (8200, 1024, 40, 1024), (4100, 1152, 300, 192), (5125, 3072, 200, 128),
+    (5125, 3072, 600, 128), (5125, 3072, 1300, 128), (4100, 320, 1500, 64), (4100, 256, 1500, 64)])
+@pytest.mark.parametrize("odd", [False, True])
+def test_gemm_bits_do_not_depend_on_the_launch(gpu, n, k, m, group, odd):
+    """A token's results have the same bits in a launch of m tokens and all n rows as in
+    one of up to 16 tokens and 64 rows, which the 16-row kernel runs."""
+    say(f"gemm bits n={n} k={k} m={m} group={group} odd {odd}")
+    w, _, s = gemv_case(n, k, 0xA70F50 + n + k, group=group)
+    x = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float16)
+    if odd:
+        w, s, x = odd_values(w, s, x)
+    got = batched_gpu(w, x, s, group)
+    rows, toks = min(n, 64), min(m, 16)
+    for t in sorted({0, (m - toks) // 2, m - toks}):
+        for r in (0, n - rows):
+            want = batched_gpu(w[r:r + rows], x[t:t + toks], s[r:r + rows], group)
+            part = got[t:t + toks, r:r + rows]
+            nan = np.isnan(want)
+            assert np.array_equal(np.isnan(part), nan), (t, r)
+            assert np.array_equal(np.where(nan, 0, part.view(np.uint16)),
+                                  np.where(nan, 0, want.view(np.uint16))), (t, r)
+            assert odd or not nan.any()
