@@ -236,15 +236,20 @@ def test_gemm_tiled_parity(gpu, n, k, m, group, y_off):
     assert np.all(err <= 0.5 * fp16_ulp(want) + bound), f"max err {err.max():.3e}"
 
 
-@pytest.mark.parametrize("fp8,m,q_off", [(False, 17, 0), (True, 40, 0), (True, 65, 0), (False, 131, 1),
-                                         (True, 300, 1), (False, 513, 0), (True, 1100, 0)])
-def test_paged_qkv_rope_append_many_tokens(gpu, fp8, m, q_off):
-    """The tiled fused form: bit for bit the batched projection followed by the
-    paged append, whole pool compared, with tokens out of range at both ends;
-    q_off: qkv rows that are not 16-byte aligned."""
-    k_in, bs, total, max_pos = 3072, 16, 96, 700
-    say(f"paged qkv rope append of {m} tokens, fp8 {fp8}")
-    w, _, s = gemv_case(QKV, k_in, 0xA70F33, group=128)
+@pytest.mark.parametrize("fp8,m,q_off,nq,k_in", [
+    (False, 17, 0, NQ, 3072), (True, 40, 0, NQ, 3072), (True, 65, 0, NQ, 3072),
+    (False, 131, 1, NQ, 3072), (True, 300, 1, NQ, 3072), (False, 513, 0, NQ, 3072),
+    (True, 1100, 0, NQ, 3072), (False, 1300, 0, NQ, 3072), (True, 1300, 1, NQ, 3072),
+    (False, 257, 0, 32, 4096), (False, 9, 1, 8, 1024), (True, 9, 0, 8, 1024), (False, 30, 0, 8, 1024),
+    (True, 30, 1, 8, 1024)])
+def test_paged_qkv_rope_append_many_tokens(gpu, fp8, m, q_off, nq, k_in):
+    """Every fused form, the tiles' (24 heads of k 3072) and the 16-row kernel's two (8 heads):
+    bit for bit the batched projection followed by the paged append, whole pool compared,
+    with tokens out of range at both ends; q_off: qkv rows that are not 16-byte aligned."""
+    bs, total, max_pos = 16, 96, 700
+    qkv_dim = (nq + 2 * NKV) * HD
+    say(f"paged qkv rope append of {m} tokens, fp8 {fp8}, {nq} query heads, k {k_in}")
+    w, _, s = gemv_case(qkv_dim, k_in, 0xA70F33, group=128)
     xs = np.random.default_rng(13).standard_normal((m, k_in)).astype(np.float16)
     r = np.random.default_rng(14)
     slots = r.permutation(total * bs)[:m].astype(np.int64)
@@ -261,15 +266,15 @@ def test_paged_qkv_rope_append_many_tokens(gpu, fp8, m, q_off):
     c, sn = oracle.rope_table(max_pos, HD, THETA)
     d_c, d_s, dx, dw, ds = up(c), up(sn), up(xs), up(w), up(s)
     d_slots, d_pos = up(slots), up(positions)
-    q1, q2 = dev.DeviceBuffer(m * QKV * 2 + 16), dev.DeviceBuffer(m * QKV * 2)
+    q1, q2 = dev.DeviceBuffer(m * qkv_dim * 2 + 16), dev.DeviceBuffer(m * qkv_dim * 2)
     st = up(np.zeros(1, np.int32))
     kv.launch_paged_qkv_rope_append(dx, k_in, m, dw, ds, k_in, q1.ptr + 2 * q_off, pools[0][1], 1,
-                                    d_slots, d_pos, d_c, d_s, max_pos, NQ, d_status=st)
-    kv.launch_w8a16_gemm_batched(dx, k_in, m, dw, ds, q2, QKV, QKV, k_in)
-    plain = q2.download(np.uint16, (m, QKV))
-    kv.launch_paged_rope_append(q2, m, pools[1][1], 1, d_slots, d_pos, d_c, d_s, max_pos, NQ)
-    got = q1.download(np.uint16)[q_off:q_off + m * QKV].reshape(m, QKV)
-    want = q2.download(np.uint16, (m, QKV))
+                                    d_slots, d_pos, d_c, d_s, max_pos, nq, d_status=st)
+    kv.launch_w8a16_gemm_batched(dx, k_in, m, dw, ds, q2, qkv_dim, qkv_dim, k_in)
+    plain = q2.download(np.uint16, (m, qkv_dim))
+    kv.launch_paged_rope_append(q2, m, pools[1][1], 1, d_slots, d_pos, d_c, d_s, max_pos, nq)
+    got = q1.download(np.uint16)[q_off:q_off + m * qkv_dim].reshape(m, qkv_dim)
+    want = q2.download(np.uint16, (m, qkv_dim))
     want[[7, m - 1]] = plain[[7, m - 1]]
     assert np.array_equal(got, want)
     assert np.array_equal(pools[0][0].download(np.uint8), pools[1][0].download(np.uint8))
