@@ -1,10 +1,11 @@
 """GPU parity of the batched paged decode forms over every GQA ratio.
 
-Batches with batch * KV heads * 2 >= CUs take the batched forms: fp16 pools the
-compact grid (workgroups mapped onto the ~512-row splits each sequence needs),
-FP8 pools the persistent grid (workgroups claiming row ranges from a counter;
+Batches with batch * KV heads * 2 >= CUs take the batched forms: the compact grid
+(workgroups mapped onto the ~512-row splits each sequence needs; small FP8 batches
+onto splits that follow the lengths), and FP8 pools whose bound is 4096 rows per
+CU or more the persistent grid (workgroups claiming row ranges from a counter;
 KV heads in pairs when their count is even, single heads when it is odd). Each
-(query heads, KV heads) shape below runs both: sampled sequences (empty,
+(query heads, KV heads) shape below runs all three: sampled sequences (empty,
 one-row, block and span boundaries, long) against the CPU oracle
 (paged_attention_f16 / paged_attention_fp8: the decode attention of
 src/kernel/tiled_attention.cu:196-269 over a block table) at the dtype's bar,
@@ -21,6 +22,7 @@ from atomflow_amd import device as dev
 from atomflow_amd import kv
 from inputs import ATOL_FP8, HD, RTOL_FP8, THETA, assert_attn_close, randn_f16, rng
 from test_gpu_paged import _sequences
+from test_gpu_persistent import persistent_bound
 
 pytestmark = pytest.mark.gpu
 
@@ -79,17 +81,18 @@ def _ref(q, host, scales, layer, table, n, bs, nq, nkv):
                                       scales[layer, 1], table, n, bs, nq, nkv, HD)
 
 
-SHAPES = [(8, 1), (9, 3), (16, 8), (64, 8)]
+SHAPES = [(8, 1), (9, 3), (8, 8), (16, 8), (32, 8), (64, 8)]
+FORMS = pytest.mark.parametrize("fp8,persistent", [(False, False), (True, False), (True, True)])
 
 
-@pytest.mark.parametrize("fp8", [False, True])
+@FORMS
 @pytest.mark.parametrize("nq,nkv", SHAPES)
-def test_batched_gqa_vs_oracle(gpu, nq, nkv, fp8):
+def test_batched_gqa_vs_oracle(gpu, nq, nkv, fp8, persistent):
     B, lengths, bm, seqs, bs, host, scales, buf, desc, d_sc = _setup(nq, nkv, fp8,
                                                                      1100 + nq + nkv + 7 * fp8)
     q_dim = nq * HD
-    say(f"batched gqa nq={nq} nkv={nkv} fp8={fp8} B={B} rows={sum(lengths)}")
-    max_len = max(lengths)
+    say(f"batched gqa nq={nq} nkv={nkv} fp8={fp8} persistent={persistent} B={B} rows={sum(lengths)}")
+    max_len = persistent_bound(B, max(lengths), persistent, nkv)
     max_blocks = (max_len + bs - 1) // bs
     tables, lens = bm.export_tables(seqs, max_blocks)
     q = randn_f16((B, q_dim), 1110 + nq)
@@ -113,14 +116,14 @@ def test_batched_gqa_vs_oracle(gpu, nq, nkv, fp8):
     bm.close()
 
 
-@pytest.mark.parametrize("fp8", [False, True])
+@FORMS
 @pytest.mark.parametrize("nq,nkv", SHAPES)
-def test_batched_gqa_fused_equals_unfused(gpu, nq, nkv, fp8):
+def test_batched_gqa_fused_equals_unfused(gpu, nq, nkv, fp8, persistent):
     B, _, bm, seqs, bs, host, scales, buf, desc, d_sc = _setup(nq, nkv, fp8,
                                                                1200 + nq + nkv + 7 * fp8)
     q_dim, kv_dim = nq * HD, nkv * HD
     qkv_w = q_dim + 2 * kv_dim
-    say(f"batched gqa fused nq={nq} nkv={nkv} fp8={fp8} B={B}")
+    say(f"batched gqa fused nq={nq} nkv={nkv} fp8={fp8} persistent={persistent} B={B}")
     plan = bm.plan_decode(seqs)
     assert not isinstance(plan, int), plan
     slots, positions, copies = plan
@@ -130,7 +133,7 @@ def test_batched_gqa_fused_equals_unfused(gpu, nq, nkv, fp8):
     bad = len(EDGE) + 2
     positions = positions.copy()
     positions[bad] = max_pos  # out of range: nothing written for this sequence
-    max_len = max(lengths) + 1
+    max_len = persistent_bound(B, max(lengths) + 1, persistent, nkv)
     max_blocks = (max_len + bs - 1) // bs
     tables, lens = bm.export_tables(seqs, max_blocks)
     c, s = oracle.rope_table(max_pos, HD, THETA)
@@ -183,8 +186,8 @@ def test_batched_gqa_fused_equals_unfused(gpu, nq, nkv, fp8):
     bm.close()
 
 
-@pytest.mark.parametrize("fp8", [False, True])
-def test_shared_blocks_policy_gives_the_same_bits(gpu, fp8):
+@FORMS
+def test_shared_blocks_policy_gives_the_same_bits(gpu, fp8, persistent):
     """AF_KV_POOL_SHARED_BLOCKS selects the kernels that read KV rows with the ordinary cache
     policy instead of non-temporal loads; only the load policy differs, so a batch whose odd
     sequences map the same blocks as their even neighbours (forks) gets the same bits either
@@ -194,9 +197,9 @@ def test_shared_blocks_policy_gives_the_same_bits(gpu, fp8):
     B, lengths, bm, seqs, bs, host, scales, buf, desc, d_sc = _setup(nq, nkv, fp8, 1300 + 7 * fp8)
     shared = kv.make_pool(buf, AF_KV_FP8_E4M3 if fp8 else AF_KV_FP16, bs, 2, nkv, HD,
                           desc.total_blocks, d_sc, flags=AF_KV_POOL_SHARED_BLOCKS)
-    say(f"shared-blocks policy fp8={fp8} B={B}")
+    say(f"shared-blocks policy fp8={fp8} persistent={persistent} B={B}")
     q_dim = nq * HD
-    max_len = max(lengths)
+    max_len = persistent_bound(B, max(lengths) + 1, persistent)
     max_blocks = (max_len + bs - 1) // bs
     tables, lens = bm.export_tables(seqs, max_blocks)
     tables[1::2], lens[1::2] = tables[0::2][: B // 2], lens[0::2][: B // 2]  # forks
@@ -223,15 +226,14 @@ def test_shared_blocks_policy_gives_the_same_bits(gpu, fp8):
     max_pos = int(positions.max()) + 2
     c, s = oracle.rope_table(max_pos, HD, THETA)
     d_c, d_s = up(c), up(s)
-    ftables, flens = bm.export_tables(seqs, (int(positions.max()) + 1 + bs - 1) // bs)
+    ftables, flens = bm.export_tables(seqs, max_blocks)
     qkv = randn_f16((B, q_dim + 2 * nkv * HD), 1320)
     res = []
     for pool in (desc, shared):
         buf.upload(host)
         d_qkv, d_o = up(qkv), dev.DeviceBuffer(B * q_dim * 2)
         kv.launch_paged_decode_fused(d_qkv, B, pool, 0, up(slots), up(positions), d_c, d_s,
-                                     max_pos, up(ftables), ftables.shape[1],
-                                     int(positions.max()) + 1, d_o, q_dim, nq, ws)
+                                     max_pos, up(ftables), max_blocks, max_len, d_o, q_dim, nq, ws)
         res.append((d_o.download(np.uint16), buf.download(np.uint8)))
     assert np.array_equal(res[0][0], res[1][0])
     assert np.array_equal(res[0][1], res[1][1])

@@ -1,8 +1,11 @@
 """GPU parity of the persistent form of batched paged decode attention.
 
 Batches of FP8 pools with the default split count (batch * KV heads * 2 >= CUs)
-run as one persistent grid whose workgroups claim items (big row ranges, then
-small ones) from a device counter. Checked here against the CPU oracle
+and a bound of 4096 rows per CU or more (batch * max_seq_len) run as one
+persistent grid whose workgroups claim items (big row ranges, then small ones)
+from a device counter. The bound, not the lengths, takes a batch there, so the
+batches here run once under the least such bound and once under their longest
+length, which takes the grid form. Checked against the CPU oracle
 (paged_attention_fp8, src/kernel/tiled_attention.cu:196-269 over a block table)
 at the FP8 bar (5e-2) and the fp16 bar, on ragged batches with empty, one-row
 and block-boundary sequences; fused decode (RoPE + append + attention) equals
@@ -54,14 +57,25 @@ def _lengths(seed, B):
     return [int(n) for n in lengths]
 
 
+def persistent_bound(B, longest, persistent, nkv=NKV):
+    """max_seq_len to pass: the least that takes the persistent form, or the longest length."""
+    cus = dev.device_info()["compute_units"]
+    least = -(-4096 * cus // B)
+    assert B * nkv * 2 >= cus and B <= 256 and longest < least
+    return least if persistent else longest
+
+
+FORMS = pytest.mark.parametrize("persistent", [True, False])
+
+
+@FORMS
 @pytest.mark.parametrize("B", [24, 64])
-def test_persistent_fp8_vs_oracle(gpu, B):
+def test_persistent_fp8_vs_oracle(gpu, B, persistent):
     lengths = _lengths(900 + B, B)
-    say(f"persistent fp8 B={B} rows={sum(lengths)}")
-    assert B * NKV * 2 >= dev.device_info()["compute_units"]  # the batched (persistent) regime
+    say(f"persistent {persistent} fp8 B={B} rows={sum(lengths)}")
     bm, seqs, P = _batch(lengths, 910 + B)
     bs = P.bs
-    max_len = max(lengths)
+    max_len = persistent_bound(B, max(lengths), persistent)
     max_blocks = (max_len + bs - 1) // bs
     tables, lens = bm.export_tables(seqs, max_blocks)
     q = randn_f16((B, Q_DIM), 920 + B)
@@ -86,22 +100,23 @@ def test_persistent_fp8_vs_oracle(gpu, B):
     bm.close()
 
 
-def test_persistent_fused_equals_unfused_and_appends(gpu):
+@FORMS
+def test_persistent_fused_equals_unfused_and_appends(gpu, persistent):
     """Fused decode (RoPE + append + attention) == append, then the unfused kernel."""
     B = 96  # several items per workgroup, so item set-up overlaps the previous tail
     lengths = _lengths(940, B)
     lengths[0] = 5  # fused decode appends to every sequence
-    say(f"persistent fused vs unfused B={B}")
+    say(f"persistent {persistent} fused vs unfused B={B}")
     bm, seqs, P = _batch(lengths, 941)
     bs = P.bs
     plan = bm.plan_decode(seqs)
     assert not isinstance(plan, int), plan
     slots, positions, copies = plan
     assert len(copies) == 0
-    max_len = max(lengths) + 1
+    max_len = persistent_bound(B, max(lengths) + 1, persistent)
     max_blocks = (max_len + bs - 1) // bs
     tables, lens = bm.export_tables(seqs, max_blocks)
-    max_pos = max_len + 1
+    max_pos = max(lengths) + 2
     c, s = oracle.rope_table(max_pos, HD, THETA)
     d_c, d_s = up(c), up(s)
     qkv = randn_f16((B, QKV), 942)
@@ -132,14 +147,15 @@ def test_persistent_fused_equals_unfused_and_appends(gpu):
     bm.close()
 
 
-def test_persistent_graph_replays(gpu):
-    """Replays of a captured persistent launch equal the eager launch (counters re-armed)."""
+@FORMS
+def test_persistent_graph_replays(gpu, persistent):
+    """Replays of a captured launch equal the eager launch (persistent: counters re-armed)."""
     B = 32
     lengths = _lengths(950, B)
-    say(f"persistent graph replays B={B}")
+    say(f"persistent {persistent} graph replays B={B}")
     bm, seqs, P = _batch(lengths, 951)
     bs = P.bs
-    max_len = max(lengths)
+    max_len = persistent_bound(B, max(lengths), persistent)
     max_blocks = (max_len + bs - 1) // bs
     tables, lens = bm.export_tables(seqs, max_blocks)
     d_q, d_t, d_l = up(randn_f16((B, Q_DIM), 952)), up(tables), up(lens)
