@@ -28,7 +28,7 @@
 //    16-byte chunks (K by row%16 for the b128 operand reads, V by 4*(row%4) for
 //    the transposing reads). They go from global memory straight into LDS
 //    (lds_dma16, no registers); later tiles' loads are issued before the current
-//    tile's matrix work: one barrier per tile.
+//    tile's matrix work: one barrier per step of one or two tiles.
 //  * Softmax is online in the log2 domain with lazy rescaling: the running max
 //    moves only when a tile's probabilities sum past 2^8 in some lane, so most
 //    tiles skip both the tile max and the O^T rescale. The row sum is taken over
@@ -50,6 +50,7 @@
 //    every piece publishes its unnormalised (o, m, l), and the last piece of the
 //    (tile, Q head) to arrive merges them in piece order.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <type_traits>
 #include <vector>
@@ -69,6 +70,9 @@ constexpr int kTileBytes = kLdsKeys * kPfHd * 2;  // one K or V tile: rows of 25
 constexpr float kPfSumLimit = 256.0f;  // per-lane tile row sum that forces a rescale
 constexpr float kPfEmptyMax = -1e30f;
 constexpr int kPfQueries = 32 * kPfWaves;  // queries per workgroup (query tile)
+// Most 64-key tiles of a workgroup that take the WIDE form: the longest workgroup of a
+// 512-token prompt (8 tiles) gains 8 % by it, 64 queries over 9 tiles lose 4 %.
+constexpr int kWideUnits = 8;
 constexpr int kPfMaxPieces = 4;            // key pieces per query tile
 constexpr int kPfMinPieceTiles = 12;       // 64-key tiles per piece, at least
 
@@ -416,21 +420,32 @@ __device__ __forceinline__ void merge_pieces(const PrefillArgs& a, float16v (&o)
     }
 }
 
-// DEEP: the scores of tile t + 1 are taken beside the softmax of tile t and every
-// operand is read before the math that needs it, over four LDS tiles and up to
-// 256 VGPRs (two workgroups per CU). Otherwise a step is one tile from scores to
-// P.V over two LDS tiles, in 168 VGPRs (three workgroups per CU, whose waves cover
-// each other). Both do the same arithmetic in the same order. Launches of few
-// workgroups are bound by a wave's own chain and take DEEP; long ones by the
-// card's power (the clock falls to 1.5 GHz as the matrix cores fill), where the
-// plain form spends less (us, DEEP / plain / the former 64-key tiles with two
-// workgroups per CU: 4096-token prompt 113 / 119 / 123, 2048 tokens behind 6144
-// 203 / 215 / 211, 8192-token prompt 416 / 404 / 444, 16384 1585 / 1521 / 1711).
-template <bool PAGED, bool FP8, bool DEEP>
+// Three forms of the key loop; all do the same arithmetic in the same order.
+//  * plain: a step is one 32-key tile from scores to P.V over two LDS tiles, in 168
+//    VGPRs (three workgroups per CU, whose waves cover each other).
+//  * DEEP: the scores of tile t + 1 are taken beside the softmax of tile t and every
+//    operand is read before the math that needs it, over four LDS tiles and up to
+//    256 VGPRs (two workgroups per CU).
+//  * WIDE: a step is two tiles, whose scores and softmax the compiler overlaps, between
+//    one wait and barrier (two workgroups per CU).
+// Launches of few workgroups are bound by a wave's own chain: short ones take WIDE
+// (few steps, little to pipeline), longer ones DEEP. Long launches are bound by the
+// matrix cores and the softmax beside them at a clock that falls as both fill, where
+// the plain form spends less. (us on MI355X, 24 query and 8 KV heads, WIDE / DEEP /
+// plain; "before" 64-key tiles, two workgroups per CU: prompt of 138 tokens 7.05 / 8.13
+// / 7.67, before 7.40; 256 tokens 9.46 / 10.54 / 10.09, before 10.11; 512 tokens 14.28 /
+// 15.48 / 15.17, before 15.78; 64 tokens behind 500 14.68 / 14.17 / 15.03, before 16.03;
+// 2048 tokens behind 6144 210 / 199 / 217, before 211; 4096-token prompt 113 / 114 / 119,
+// before 123; 8192 414 / 411 / 404, before 433. FP8 pool: 138 tokens 7.76 / 8.77, before
+// 7.96; 512 16.5 / 17.5, before 17.6; 2048 behind 6144 233 / 222, before 237.)
+enum Form { kPlain, kDeep, kWide };
+template <bool PAGED, bool FP8, Form FORM>
 __device__ __forceinline__ void prefill_body(const PrefillArgs& args) {
     PrefillArgs a = args;
     constexpr int kQueries = 32 * kPfWaves;  // per workgroup
-    constexpr int kStages = DEEP ? 4 : 2;        // LDS tiles of K, then of V
+    constexpr bool DEEP = FORM == kDeep;
+    constexpr int kStages = FORM == kPlain ? 2 : 4;  // LDS tiles of K, then of V
+    constexpr int kPer = FORM == kWide ? 2 : 1;      // tiles per step
     constexpr int kVBase = kStages * kTileBytes;
     __shared__ __align__(16) char s_lds[2 * kStages * kTileBytes];
 
@@ -547,32 +562,39 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& args) {
     const char* kb = reinterpret_cast<const char*>(a.k) + size_t(kvh) * kPfHd * kElem;
     const char* vb = reinterpret_cast<const char*>(a.v) + size_t(kvh) * kPfHd * kElem;
     const uint32_t lds0 = lds_address(s_lds);
-    Fp8Tile f8;
-    // Fetches tile kt: into `stage` (fp16), or into f8 for fp8_store. The plain
-    // form reads the block-table entry a step ahead; DEEP reads it here: with a
+    Fp8Tile f8[kPer];
+    // Fetches tile kt: into `stage` (fp16), or into an f8 for fp8_store. The plain
+    // form reads the block-table entry a step ahead; the others read it here: with a
     // scalar load outstanding, every wait for an LDS operand waits for all of
-    // them (five 512-token chunks with their projection 212 us, a step ahead 219).
-    int entry = DEEP ? 0 : tile_entry<PAGED>(a, kt_lo, wave);
+    // them (DEEP, five 512-token chunks with their projection 212 us, a step ahead 219).
+    constexpr bool kEntryAhead = FORM == kPlain;
+    int entry = kEntryAhead ? tile_entry<PAGED>(a, kt_lo, wave) : 0;
     auto fetch = [&](int kt, int stage) __attribute__((always_inline)) {
         const RowSource src =
-            tile_rows<PAGED>(a, kt, wave, DEEP ? tile_entry<PAGED>(a, kt, wave) : entry);
+            tile_rows<PAGED>(a, kt, wave, kEntryAhead ? entry : tile_entry<PAGED>(a, kt, wave));
         if constexpr (FP8) {
-            fp8_load(kb, vb, a.kv_row_bytes, src, lane, f8);
+            fp8_load(kb, vb, a.kv_row_bytes, src, lane, f8[stage % kPer]);
         } else {
             dma_rows<true>(kb, a.kv_row_bytes, src, wave, lane, lds0 + stage * kTileBytes);
             dma_rows<false>(vb, a.kv_row_bytes, src, wave, lane,
                             lds0 + kVBase + stage * kTileBytes);
         }
     };
-    constexpr int kAhead = kStages - 1;  // tiles fetched ahead of the current one
+    auto store = [&](int stage) __attribute__((always_inline)) {
+        if constexpr (FP8)
+            fp8_store(s_lds + stage * kTileBytes, s_lds + kVBase + stage * kTileBytes, tid,
+                      f8[stage % kPer]);
+    };
+    constexpr int kAhead = kStages - kPer;  // tiles fetched ahead of the current one
 #pragma unroll
-    for (int i = 0; i < (DEEP ? kAhead : 1); ++i) {
-        if (kt_lo + i < n_kt) {
-            fetch(kt_lo + i, i);
-            if constexpr (FP8)
-                fp8_store(s_lds + i * kTileBytes, s_lds + kVBase + i * kTileBytes, tid, f8);
-        }
-        if constexpr (!DEEP) entry = tile_entry<PAGED>(a, min(kt_lo + 1, n_kt - 1), wave);
+    for (int i = 0; i < kAhead; i += kPer) {
+#pragma unroll
+        for (int j = i; j < i + kPer; ++j)
+            if (kt_lo + j < n_kt) fetch(kt_lo + j, j);
+#pragma unroll
+        for (int j = i; j < i + kPer; ++j)
+            if (kt_lo + j < n_kt) store(j);
+        if constexpr (kEntryAhead) entry = tile_entry<PAGED>(a, min(kt_lo + 1, n_kt - 1), wave);
     }
     if (a.cos_t) {  // packed partials with RoPE (wave-uniform)
         // Whole 32-bit words in and out: two fp16 elements per word, low half
@@ -606,9 +628,9 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& args) {
         }
     }
 
-    // Per-lane LDS operand offsets; the buffer, the key block and the key step
-    // are added as immediates.
-    //  K: row col (+32 for keys 32..63), chunk 2s+hi.
+    // Per-lane LDS operand offsets; the stage and the key step are added as
+    // immediates.
+    //  K: row col, chunk 2s+hi.
     //  V^T: lane l of 16-lane group G reads row K0 + (l%16)/4 at d = 32db +
     //  16(G%2) + 4(l%4), K0 = 16j + 8u + 4hi (u: first / second four slots).
     uint32_t ka[8], va[4];
@@ -681,27 +703,33 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& args) {
         const char* p = s_lds + stage * kTileBytes + va[db] + 16 * jj * 256;  // va[]: the V region
         return lds_vt(p, p + 8 * 256);
     };
-    // Tile kt + kAhead goes to the stage that the barrier before has freed.
+    // The tiles kAhead after kt, .. go to the stages that the barrier before has freed.
     auto fetch_ahead = [&](int kt, int stage) __attribute__((always_inline)) {
-        if (kt + kAhead < n_kt) fetch(kt + kAhead, stage);
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+            if (kt + kAhead + j < n_kt) fetch(kt + kAhead + j, stage + j);
     };
     auto end_step = [&](int kt, int stage) __attribute__((always_inline)) {
-        if constexpr (FP8)
-            if (kt + kAhead < n_kt)
-                fp8_store(s_lds + stage * kTileBytes, s_lds + kVBase + stage * kTileBytes, tid, f8);
-        if constexpr (PAGED && !DEEP) entry = tile_entry<PAGED>(a, min(kt + 2, n_kt - 1), wave);
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+            if (kt + kAhead + j < n_kt) store(stage + j);
+        if constexpr (PAGED && kEntryAhead)
+            entry = tile_entry<PAGED>(a, min(kt + 2, n_kt - 1), wave);
     };
 
     if constexpr (!DEEP) {
+        // Tiles kt .. kt + kPer - 1, in stages S ..
         auto step = [&](int kt, auto stage_c) __attribute__((always_inline)) {
             constexpr int S = decltype(stage_c)::value;
             // This wave's tile loads have landed in LDS; the barrier covers the
-            // others' and frees the other stage (read in the previous step).
+            // others' and frees the other stages (read in the previous step).
             lds_dma_wait();
             __syncthreads();
-            fetch_ahead(kt, S ^ 1);
-            if (kt * kLdsKeys < w_keys) {  // wave-uniform
-                const char* ks = s_lds + S * kTileBytes;
+            fetch_ahead(kt, S ^ kPer);
+#pragma unroll
+            for (int j = 0; j < kPer; ++j) {
+                if ((kt + j) * kLdsKeys >= w_keys || (kPer > 1 && kt + j >= n_kt)) break;  // wave-uniform
+                const char* ks = s_lds + (S + j) * kTileBytes;
                 float16v sacc;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sacc[r] = 0.0f;
@@ -709,22 +737,22 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& args) {
                 for (int s = 0; s < 8; ++s)
                     sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(lds_half8(ks + ka[s]), qf[s],
                                                                   sacc, 0, 0, 0);
-                mask_scores(kt, sacc);
+                mask_scores(kt + j, sacc);
                 half8 pj[2];
                 softmax(sacc, pj);
 #pragma unroll
                 for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
                     for (int db = 0; db < 4; ++db)
-                        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(value_operand(S, jj, db),
+                        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(value_operand(S + j, jj, db),
                                                                        pj[jj], o[db], 0, 0, 0);
             }
-            end_step(kt, S ^ 1);
+            end_step(kt, S ^ kPer);
         };
         int kt = kt_lo;
-        for (; kt + 2 <= n_kt; kt += 2) {
+        for (; kt + kPer < n_kt; kt += 2 * kPer) {
             step(kt, std::integral_constant<int, 0>{});
-            step(kt + 1, std::integral_constant<int, 1>{});
+            step(kt + kPer, std::integral_constant<int, kPer>{});
         }
         if (kt < n_kt) step(kt, std::integral_constant<int, 0>{});
     } else {
@@ -826,31 +854,42 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& args) {
         }
 }
 
-// The plain form (FP8 pools: DEEP always).
+// The plain form (FP8 pools: DEEP).
 template <bool PAGED, bool FP8>
 __global__ __launch_bounds__(kPfThreads, FP8 ? 2 : 3) void prefill_attention_kernel(
     const PrefillArgs a) {
-    prefill_body<PAGED, FP8, FP8>(a);
+    prefill_body<PAGED, FP8, FP8 ? kDeep : kPlain>(a);
 }
 
 template <bool PAGED>
 __global__ __launch_bounds__(kPfThreads, 2) void prefill_deep_kernel(const PrefillArgs a) {
-    prefill_body<PAGED, false, true>(a);
+    prefill_body<PAGED, false, kDeep>(a);
+}
+
+template <bool PAGED, bool FP8>
+__global__ __launch_bounds__(kPfThreads, 2) void prefill_wide_kernel(const PrefillArgs a) {
+    prefill_body<PAGED, FP8, kWide>(a);
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Launches `wgs` workgroups: FP8 pools always DEEP, fp16 up to about four
-// workgroups per CU (see the kernel).
-int launch_grid(const PrefillArgs& a, int wgs, hipStream_t stream) {
+// Launches `wgs` workgroups of at most `units` 64-key tiles each (see the kernel).
+int launch_grid(const PrefillArgs& a, int wgs, int units, hipStream_t stream) {
     const dim3 grid(wgs), block(kPfThreads);
+    const bool wide = units <= kWideUnits;
     const bool deep = wgs <= 4 * device_compute_units();
-    if (a.scales)
+    if (a.scales && wide)
+        hipLaunchKernelGGL((prefill_wide_kernel<true, true>), grid, block, 0, stream, a);
+    else if (a.scales)
         hipLaunchKernelGGL((prefill_attention_kernel<true, true>), grid, block, 0, stream, a);
+    else if (a.table && wide)
+        hipLaunchKernelGGL((prefill_wide_kernel<true, false>), grid, block, 0, stream, a);
     else if (a.table && deep)
         hipLaunchKernelGGL((prefill_deep_kernel<true>), grid, block, 0, stream, a);
     else if (a.table)
         hipLaunchKernelGGL((prefill_attention_kernel<true, false>), grid, block, 0, stream, a);
+    else if (wide)
+        hipLaunchKernelGGL((prefill_wide_kernel<false, false>), grid, block, 0, stream, a);
     else if (deep)
         hipLaunchKernelGGL((prefill_deep_kernel<false>), grid, block, 0, stream, a);
     else
@@ -861,7 +900,9 @@ int launch_grid(const PrefillArgs& a, int wgs, hipStream_t stream) {
 
 int launch_prefill(PrefillArgs a, hipStream_t stream) {
     a.n_tiles = ceil_div(a.n, 32 * kPfWaves);
-    return launch_grid(a, a.n_tiles * a.n_q_heads * std::max(a.n_pieces, 1), stream);
+    // of the last query tile, uncut
+    const int units = ceil_div(int(std::min<int64_t>(int64_t(a.p0) + a.n, a.kv_len)), kPfKeys);
+    return launch_grid(a, a.n_tiles * a.n_q_heads * std::max(a.n_pieces, 1), units, stream);
 }
 
 }  // namespace
@@ -898,7 +939,8 @@ int launch_prefix_partials(const PrefixPartialArgs& p, hipStream_t stream) {
     a.sin_t = p.sin_t;
     a.positions = p.positions;
     a.max_pos = p.max_pos;
-    return launch_grid(a, a.n_tiles * a.n_q_heads * p.key_splits, stream);
+    const int units = ceil_div(ceil_div(p.prefix_len, kPfKeys), p.key_splits);
+    return launch_grid(a, a.n_tiles * a.n_q_heads * p.key_splits, units, stream);
 }
 
 // Key-tiles per piece for a launch whose query tiles need units[i] 64-key
@@ -1273,7 +1315,8 @@ static int prefill_batched(const void* q, int q_stride, const af_kv_pool* pool, 
             carve_records(a, workspace, n_groups, max_pieces);
         }
     }
-    return launch_grid(a, n_tiles * n_q_heads, static_cast<hipStream_t>(stream));
+    // (the chunks' lengths are on the device)
+    return launch_grid(a, n_tiles * n_q_heads, INT_MAX, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int af_paged_prefill_attention_batched(

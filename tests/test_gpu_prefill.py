@@ -380,6 +380,50 @@ def test_prefill_forms_give_the_same_bits(gpu, bs, p0, kv_len):
             assert np.array_equal(got, want[first:first + rows]), (first, rows, paged)
 
 
+@pytest.mark.parametrize("nq,nkv,pool", [(24, 8, None), (24, 8, "fp16"), (24, 8, "fp8"),
+                                         (9, 3, "fp16"), (8, 1, "fp8"), (64, 8, None)])
+def test_prefill_short_form_gives_the_same_bits(gpu, nq, nkv, pool):
+    """A workgroup of at most 512 keys takes a loop of its own over the same arithmetic: the
+    queries before row `end` of a 700-token prompt, launched alone with end keys, give the
+    bits they have in the whole launch, at every edge of the 32-key tiles and their pairs."""
+    n, bs = 700, 16
+    say(f"prefill short form nq={nq} nkv={nkv} pool={pool}")
+    q_dim, kv_dim, blocks = nq * HD, nkv * HD, (n + bs - 1) // bs
+    table = rng(nq + nkv).permutation(blocks + 3)[:blocks].astype(np.int32)
+    r = rng(0xA70F7A + nq)
+    d_t = up(table)
+    if pool == "fp8":
+        host = r.integers(0, 256, (2, (blocks + 3) * bs, kv_dim), dtype=np.uint8)
+        host[(host & 0x7F) == 0x7F] = 0
+        d_sc = up(r.uniform(0.004, 0.01, (1, 2, nkv)).astype(np.float32))
+    else:
+        host, d_sc = randn_f16((2, (blocks + 3) * bs, kv_dim), 0xA70F7B + nq), None
+    d_kv = up(host)
+    desc = kv.make_pool(d_kv, atomflow_amd.AF_KV_FP8_E4M3 if pool == "fp8" else atomflow_amd.AF_KV_FP16,
+                        bs, 1, nkv, HD, blocks + 3, d_sc)
+    d_k, d_v = up(host[0]), up(host[1])
+    d_q = up(randn_f16((n, q_dim), 0xA70F7C + nq))
+    d_o = dev.DeviceBuffer(n * q_dim * 2)
+
+    def launch(p0, rows):
+        first = d_q.ptr + p0 * q_dim * 2
+        if pool:
+            kv.launch_paged_prefill_attention(first, q_dim, desc, 0, d_t, blocks, p0, rows, p0 + rows,
+                                              d_o, q_dim, nq)
+        else:
+            kv.launch_prefill_attention(first, q_dim, d_k, d_v, d_o, q_dim, p0, rows, p0 + rows,
+                                        p0 + rows, nq, nkv, HD)
+        return d_o.download(np.uint16)[:rows * q_dim].reshape(rows, q_dim).copy()
+
+    want = launch(0, n)
+    assert np.all(np.isfinite(want.view(np.float16)))
+    for end in (1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 160, 255, 256, 257, 448, 511, 512,
+                513, 577):
+        for rows in sorted({1, min(end, 40), end}):
+            got = launch(end - rows, rows)
+            assert np.array_equal(got, want[end - rows:end]), (end, rows)
+
+
 def test_paged_prefill_rejects_bad_arguments(gpu):
     say("paged prefill argument checks")
     lib = atomflow_amd.lib()
