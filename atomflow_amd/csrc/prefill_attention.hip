@@ -750,11 +750,12 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& args) {
             end_step(kt, S ^ kPer);
         };
         int kt = kt_lo;
-        for (; kt + kPer < n_kt; kt += 2 * kPer) {
+        for (; kt + 2 * kPer <= n_kt; kt += 2 * kPer) {
             step(kt, std::integral_constant<int, 0>{});
             step(kt + kPer, std::integral_constant<int, kPer>{});
         }
         if (kt < n_kt) step(kt, std::integral_constant<int, 0>{});
+        if (kPer > 1 && kt + kPer < n_kt) step(kt + kPer, std::integral_constant<int, kPer>{});
     } else {
         auto scores = [&](int stage, float16v& sacc) __attribute__((always_inline)) {
             const char* ks = s_lds + stage * kTileBytes;
