@@ -189,10 +189,6 @@ struct AttnArgs {
     // the CACHED kernels, which read KV rows with the ordinary cache policy
     // instead of non-temporal loads.
     int32_t cached_rows;
-    // Compact grid of up to 64 sequences, target_splits > 0: every sequence's span
-    // is the smallest (at least kMinSpan, at most span_tokens) with which the
-    // batch has at most target_splits splits (see adaptive_span).
-    int32_t target_splits;
 };
 
 template <int HD, bool FP8>
@@ -446,6 +442,14 @@ __device__ __forceinline__ int grid_splits(const AttnArgs& a, int L, int step_ro
     return max(1, min(a.num_splits, (total_steps + span_steps - 1) / span_steps));
 }
 
+// ceil(x / y) for x < 5 10^6, inv = 1 / y on v_rcp_f32: the product is then less than
+// 1 / y off the quotient, so its integer part is the floor, the ceiling, or (exact
+// multiples) one below, which is mended.
+__device__ __forceinline__ unsigned ceil_quotient(unsigned x, unsigned y, float inv) {
+    const unsigned q = unsigned(float(x) * inv);
+    return q + (q * y < x ? 1u : 0u);
+}
+
 // Span of a small batch, in workgroup steps; lane s holds sequence s's length L
 // (any value past the batch). Wave-uniform. A launch whose (sequence, head) pairs
 // are few can give every split a CU of its own, and it ends with its longest
@@ -461,26 +465,43 @@ __device__ __forceinline__ int grid_splits(const AttnArgs& a, int L, int step_ro
 // sequences of 768 .. 12288 rows 57.7 / 49.4 fp16 and 71.0 / 38.0 FP8, 12 of 256
 // .. 4096 40.9 / 33.1 and 54.8 / 30.3, 15 of 512 .. 8192 71.1 / 60.8 and 89.7 /
 // 43.1.)
+// Cutting a sequence costs a merge, about what kMergeRows more rows in a split take: if
+// the longest has no more than that past the span, all stay whole (attention alone, 16
+// sequences of 256 rows: whole 8.0 us fp16 and 11.1 FP8, in 64-row splits 9.4 and 12.3;
+// 8 FP8 ones of 384: 13.6 and 11.9). And a record's merge costs about what 9 rows do, so
+// a span is at least kSpanRoot sqrt(rows) rows (2 FP8 sequences of 2048 rows in 32 / 16 /
+// 8 splits 16.0 / 13.7 / 15.0 us). The arithmetic is on every launch's way, so its
+// divisions are products with reciprocals; where it changes nothing it costs 0.2 to 0.4
+// us against one fixed split count (2 fp16 sequences of 512 rows under a bound of 16384
+// rows 9.0 us and 8.7; 8 of 4096 25.3 and 24.9).
+constexpr unsigned kMergeRows = 220;
+constexpr float kSpanRoot = 3.0f;
 __device__ __forceinline__ int adaptive_span(const AttnArgs& a, int L, int step_rows) {
     const bool seq = int(threadIdx.x & 63) < a.batch;
     const unsigned steps = seq ? unsigned(max(L, 0) + step_rows - 1) / unsigned(step_rows) : 0u;
+    const unsigned most = __builtin_amdgcn_readlane(wave_inclusive_max(int(steps)), 63);
     const unsigned all = __builtin_amdgcn_readlane(wave_inclusive_sum(int(steps)), 63);
-    const unsigned lo = max(1, kMinSpan / step_rows), hi = max(1, a.span_tokens / step_rows);
-    const unsigned target = a.target_splits;
+    const unsigned merge = kMergeRows / step_rows;
+    if (most <= kMinSpan / step_rows + merge) return int(max(1u, most));
+    const unsigned hi = max(1, a.span_tokens / step_rows);
+    const unsigned root = unsigned(kSpanRoot * __builtin_amdgcn_sqrtf(float(most * step_rows)));
+    const unsigned lo = max(unsigned(kMinSpan), root) / unsigned(step_rows);
+    const unsigned target = a.compact & 0xffff, each = unsigned(a.compact) >> 16;
     unsigned t = target, span;
-    if (!__builtin_amdgcn_ballot_w64(steps * 8 * a.batch > all * 9)) {  // nearly equal
-        const unsigned most = __builtin_amdgcn_readlane(wave_inclusive_max(int(steps)), 63);
-        t = target / a.batch;
-        return int(min(max((most + t - 1) / t, lo), hi));
+    if (most * 8 * a.batch <= all * 9) {  // nearly equal
+        span = max(ceil_quotient(most, each, __builtin_amdgcn_rcpf(float(each))), lo);
+    } else {
+        for (int attempt = 0;; ++attempt) {
+            span = max(ceil_quotient(all, t, __builtin_amdgcn_rcpf(float(t))), lo);
+            if (attempt == 3) break;
+            const unsigned own =
+                seq ? max(1u, ceil_quotient(steps, span, __builtin_amdgcn_rcpf(float(span)))) : 0u;
+            const unsigned count = __builtin_amdgcn_readlane(wave_inclusive_sum(int(own)), 63);
+            if (count <= target) break;
+            t = attempt == 2 ? target - a.batch : max(t - min(t, count - target), target - a.batch);
+        }
     }
-    for (int attempt = 0;; ++attempt) {
-        span = max((all + t - 1) / t, lo);
-        if (attempt == 3) break;
-        const unsigned own = seq ? max(1u, (steps + span - 1) / span) : 0u;
-        const unsigned count = __builtin_amdgcn_readlane(wave_inclusive_sum(int(own)), 63);
-        if (count <= target) break;
-        t = attempt == 2 ? target - a.batch : max(t - min(t, count - target), target - a.batch);
-    }
+    if (most <= span + merge) span = max(span, most);
     return int(min(span, hi));
 }
 
@@ -1280,7 +1301,7 @@ __device__ __forceinline__ void decode_attn_body(const AttnArgs& a) {
             // wave-wide scan and a ballot; no LDS round trip, no barrier).
             const int lane = tid & 63;
             const int Lb = lane < a.batch ? length(lane) : 0;
-            if (a.target_splits > 0) span_steps = adaptive_span(a, Lb, STEP);
+            if (a.compact > 1) span_steps = adaptive_span(a, Lb, STEP);
             const int n = lane < a.batch ? grid_splits(a, Lb, STEP, span_steps) : 0;
             const int incl = wave_inclusive_sum(n);
             if (id >= int64_t(__builtin_amdgcn_readlane(incl, 63)) * nhw) return;
@@ -1844,7 +1865,8 @@ int device_compute_units() {
 // Batches with at least half a (sequence, KV head) pair per CU balance the work
 // per workgroup: every split covers about kBatchSpan tokens, so a sequence's
 // split count follows its length. Smaller launches split every sequence the
-// same way to fill the CUs.
+// same way to fill the CUs, except the paged ones of 2 to 64 sequences that take
+// spans of their own (adaptive_span).
 int default_span(int batch, int n_kv_heads) {
     return int64_t(batch) * n_kv_heads * 2 >= device_compute_units() ? kBatchSpan : kMinSpan;
 }
@@ -2148,6 +2170,7 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
     const int suffix_max = std::max(max_seq_len - prefix.len, 1);
     const int min_sp = min_splits_for_table(std::max(suffix_max, std::min(prefix.len, max_seq_len)), bs);
     int span = kMinSpan;
+    const int nhw = fp8 && nkv % 2 == 0 ? nkv / 2 : nkv;  // workgroups per (sequence, split)
     bool persistent_ok = false;  // the default partition of a batch may run persistent
     bool adaptive_ok = false;    // ... or span-adaptive
     if (num_splits <= 0) {
@@ -2161,9 +2184,10 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
         // / 576, 64 of the same 325 / 313, 128 of 512 .. 8192 242 / 236; below,
         // 96 of 512 .. 8192 183 / 195, 48 of 8192 102 / 121, 64 of 512 .. 8192
         // 130 / 147, 128 of 128 .. 2048 86 / 100, 96 of 64 .. 1024 51 / 66.)
-        persistent_ok = fp8 && span == kBatchSpan && prefix.len == 0 && hd == 128 &&
-                        batch <= kMaxPersistBatch &&
-                        int64_t(batch) * max_seq_len >= int64_t(4096) * device_compute_units();
+        const bool fp8_batch = fp8 && span == kBatchSpan && prefix.len == 0 && hd == 128 &&
+                               batch <= kMaxPersistBatch;
+        persistent_ok =
+            fp8_batch && int64_t(batch) * max_seq_len >= int64_t(4096) * device_compute_units();
         adaptive_ok = prefix.len == 0 && batch > 1 && batch <= kWave && !persistent_ok;
         if (prefix.len > 0 && span == kBatchSpan) {
             // Batched suffixes behind a shared prefix are short: splits of up to
@@ -2191,17 +2215,20 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
     // Small batches: spans that follow the lengths (adaptive_span), about one
     // workgroup per CU, when a (sequence, workgroup column) pair has two CUs or
     // more and there are rows to spread (shorter launches gain less than the
-    // span's arithmetic costs, 0.3 us). (Three for four CUs: 8 sequences
-    // of 768 .. 12288 fp16 rows 51.9 us against 49.1.) As many records as the
-    // workspace holds, never fewer than the fixed count needs. (Row sums stay
-    // within 31 bits.)
+    // span's arithmetic costs, 0.2 to 0.4 us; so do those of up to about 320 rows that
+    // the fixed count leaves whole). (Three for four CUs: 8 sequences
+    // of 768 .. 12288 fp16 rows 51.9 us against 49.1. At two, the longest split can be
+    // half as long again as the mean: 16 fp16 sequences of 4096 rows 51.6 us with spans
+    // of 512, 45.1 so; of 1024 .. 16384 rows, three draws, 101 / 95, 141 / 138 and 129 /
+    // 152.) As many records as the
+    // workspace holds, never fewer than the fixed count needs. (Up to 2^26 rows: the
+    // steps, at least 16 rows each, stay within ceil_quotient's range.)
     int target_splits = 0;
     int64_t grid = int64_t(batch) * num_splits * nkv;
     const int cus = device_compute_units();
-    const int nhw = fp8 && nkv % 2 == 0 ? nkv / 2 : nkv;  // workgroups per (sequence, split)
     const int64_t rows = int64_t(batch) * max_seq_len;
     if (adaptive_ok && int64_t(batch) * nhw * 2 <= cus && rows > (fp8 ? 2048 : 8192) &&
-        rows < INT32_MAX / 2) {
+        !(num_splits == 1 && max_seq_len <= 320) && rows < (int64_t(1) << 26)) {
         span = max_span_for_table(bs) / kStepTokens * kStepTokens;  // whole steps
         target_splits = cus / nhw;
         int n = std::min({target_splits, kMaxSplits, ceil_div(max_seq_len, kMinSpan)});
@@ -2243,7 +2270,6 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
     a.n_kv_heads = nkv;
     a.num_splits = num_splits;
     a.span_tokens = span;
-    a.target_splits = target_splits;
     a.qk_scale = qk_scale_for(hd);
     a.scales = fp8 ? pool->scales + size_t(layer) * 2 * nkv : nullptr;
     a.part_o = w.part_o;
@@ -2257,7 +2283,8 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
     // (Only batched launches without a shared prefix: the shared-prefix form's
     // short suffix splits measured slower with the length scan, 64 forks of
     // 2048 rows 55.2 against 51.9 us.)
-    a.compact = (span == kBatchSpan || target_splits > 0) && pre == 0 && batch <= kThreads;
+    a.compact = span >= kBatchSpan && pre == 0 && batch <= kThreads;
+    if (target_splits > 0) a.compact = target_splits | (target_splits / batch) << 16;
     if (grid > INT32_MAX) return AF_ERR_UNSUPPORTED;
     if (pre > 0) {  // the prefix's partials first: records 0 .. pre-1
         PrefixPartialArgs pp{};

@@ -419,9 +419,10 @@ _SPAN_LENGTHS = {  # lengths of a small batch whose spans follow them
 }
 
 
-@pytest.mark.parametrize("fp8,B,L", [(False, 2, 4097), (False, 2, 4096), (False, 16, 1025),
-                                     (False, 17, 1025), (True, 2, 4097), (True, 32, 300),
-                                     (True, 33, 300)])
+@pytest.mark.parametrize("fp8,B,L", [(False, 2, 4097), (False, 2, 4096), (False, 15, 1025),
+                                     (False, 16, 1025), (False, 17, 1025), (True, 2, 4097),
+                                     (True, 32, 300), (True, 33, 300), (True, 32, 600),
+                                     (True, 33, 600), (True, 8, 401), (True, 8, 400)])
 @pytest.mark.parametrize("kind", sorted(_SPAN_LENGTHS))
 def test_paged_small_batch_spans(gpu, fp8, B, L, kind):
     """Default splits of small batches, each side of the rule's edges, in a workspace of full and
