@@ -2188,6 +2188,15 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
                                batch <= kMaxPersistBatch;
         persistent_ok =
             fp8_batch && int64_t(batch) * max_seq_len >= int64_t(4096) * device_compute_units();
+        if (fp8_batch && !persistent_ok &&
+            int64_t(batch) * nhw >= 2 * int64_t(device_compute_units())) {
+            // Two workgroups per CU without a cut: longer splits, fewer merges (us,
+            // persistent / spans of 512 / 1024: 128 sequences of 1024 rows 58.6 / 65.0 /
+            // 50.0, 192 of 2048 157 / 163 / 151, 128 of 64 .. 1024 53.7 / 39.0 / 37.4;
+            // with fewer sequences the ragged ones lose: 96 of 64 .. 1024 36.4 / 37.3).
+            span = 2 * kBatchSpan;
+            num_splits = std::max(std::min(ceil_div(suffix_max, span), kMaxSplits), min_sp);
+        }
         adaptive_ok = prefix.len == 0 && batch > 1 && batch <= kWave && !persistent_ok;
         if (prefix.len > 0 && span == kBatchSpan) {
             // Batched suffixes behind a shared prefix are short: splits of up to

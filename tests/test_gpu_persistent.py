@@ -238,3 +238,56 @@ def test_persistent_bound_vs_oracle(gpu, below):
     finally:
         g.destroy()
     bm.close()
+
+
+def test_grid_form_of_a_large_batch_vs_oracle(gpu):
+    """FP8 batches with two workgroups per CU and a bound below the persistent form's: spans
+    of 1024 rows, at their edges; fused equals unfused, replays equal the eager launch."""
+    cus = dev.device_info()["compute_units"]
+    B = max(128, -(-4 * cus // NKV))
+    edges = [1, 5, 511, 512, 513, 1022, 1023, 1024, 1025, 2046, 2047, 2048, 2049]
+    lengths = edges + [int(n) for n in rng(980).integers(1, 130, B - len(edges))]
+    bound = max(lengths) + 1
+    assert B * NKV // 2 >= 2 * cus and B <= 256 and B * bound < 4096 * cus
+    say(f"grid form B={B} bound={bound}")
+    bm, seqs, P = _batch(lengths, 981)
+    bs = P.bs
+    slots, positions, copies = bm.plan_decode(seqs)
+    max_blocks = (bound + bs - 1) // bs
+    tables, lens = bm.export_tables(seqs, max_blocks)
+    max_pos = bound + 1
+    c, s = oracle.rope_table(max_pos, HD, THETA)
+    d_c, d_s = up(c), up(s)
+    d_qkv, d_t, d_l = up(randn_f16((B, QKV), 982)), up(tables), up(lens)
+    d_sl, d_p = up(slots), up(positions)
+    d_o1, d_o2 = dev.DeviceBuffer(B * Q_DIM * 2), dev.DeviceBuffer(B * Q_DIM * 2)
+    ws = kv.AttentionWorkspace(B, NQ, NKV, HD, 0)
+    stream = dev.Stream()
+    kv.launch_paged_decode_fused(d_qkv, B, P.desc, 1, d_sl, d_p, d_c, d_s, max_pos, d_t,
+                                 max_blocks, bound, d_o1, Q_DIM, NQ, ws, stream=stream)
+
+    def launch():
+        kv.launch_paged_attention(d_qkv, QKV, P.desc, 1, d_t, max_blocks, d_l, B, bound, d_o2,
+                                  Q_DIM, NQ, ws, stream=stream)
+
+    launch()
+    stream.sync()
+    got = d_o2.download(np.float16, (B, Q_DIM)).copy()
+    assert np.array_equal(bits(d_o1.download(np.float16, (B, Q_DIM))), bits(got))
+    q, pool = d_qkv.download(np.float16, (B, QKV))[:, :Q_DIM], P.download()
+    for b in list(range(len(edges))) + [B - 1]:
+        ref = oracle.paged_attention_fp8(q[b], pool[1, 0], pool[1, 1], P.scales[1, 0],
+                                         P.scales[1, 1], tables[b], lengths[b] + 1, bs, NQ, NKV, HD)
+        assert_attn_close(got[b], ref, what=f"seq {b}")
+    g = dev.Graph.capture(stream, launch)
+    try:
+        for i in range(3):
+            d_o2.upload(np.zeros(B * Q_DIM, np.float16))
+            g.launch(stream)
+            stream.sync()
+            assert np.array_equal(bits(d_o2.download(np.float16, (B, Q_DIM))), bits(got)), i
+            launch()
+            stream.sync()
+    finally:
+        g.destroy()
+    bm.close()
