@@ -2173,6 +2173,7 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
     const int nhw = fp8 && nkv % 2 == 0 ? nkv / 2 : nkv;  // workgroups per (sequence, split)
     bool persistent_ok = false;  // the default partition of a batch may run persistent
     bool adaptive_ok = false;    // ... or span-adaptive
+    int min_records = 0;         // the default count's records, asked of the workspace all the same
     if (num_splits <= 0) {
         num_splits = std::max(default_splits_for(suffix_max, batch, nkv, false), min_sp);
         span = default_span(batch, nkv);
@@ -2195,6 +2196,7 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
             // 50.0, 192 of 2048 157 / 163 / 151, 128 of 64 .. 1024 53.7 / 39.0 / 37.4;
             // with fewer sequences the ragged ones lose: 96 of 64 .. 1024 36.4 / 37.3).
             span = 2 * kBatchSpan;
+            min_records = num_splits;
             num_splits = std::max(std::min(ceil_div(suffix_max, span), kMaxSplits), min_sp);
         }
         adaptive_ok = prefix.len == 0 && batch > 1 && batch <= kWave && !persistent_ok;
@@ -2219,7 +2221,8 @@ static int paged_attention(void* q, int q_stride, const af_kv_pool* pool, int la
         if (num_splits + pre > kMaxSplits) return AF_ERR_OUT_OF_RANGE;
     }
     int rec_stride = num_splits + pre;
-    if (!workspace || workspace_bytes < attn_workspace_bytes(batch, n_q_heads, hd, rec_stride))
+    if (!workspace || workspace_bytes < attn_workspace_bytes(batch, n_q_heads, hd,
+                                                             std::max(rec_stride, min_records)))
         return AF_ERR_WORKSPACE;
     // Small batches: spans that follow the lengths (adaptive_span), about one
     // workgroup per CU, when a (sequence, workgroup column) pair has two CUs or

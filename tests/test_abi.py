@@ -121,6 +121,23 @@ def test_shared_prefix_argument_checks_without_gpu():
     assert lib.af_kv_pool_bytes(ctypes.byref(shared)) == lib.af_kv_pool_bytes(ctypes.byref(pool))
 
 
+@pytest.mark.parametrize("batch,rows", [(128, 513), (128, 1024), (128, 8000), (200, 1025)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_paged_attention_asks_the_default_split_count_of_its_workspace(fp8, batch, rows):
+    """A batched launch takes one record per 512 rows of max_seq_len, whatever spans its form
+    cuts: a workspace one byte short of that is refused, before any device call."""
+    import ctypes
+    from atomflow_amd import kv
+    lib = atomflow_amd.lib()
+    fake = 0x10000  # never dereferenced
+    pool = kv.make_pool(fake, atomflow_amd.AF_KV_FP8_E4M3 if fp8 else atomflow_amd.AF_KV_FP16, 16, 2,
+                        8, 128, 1000, scales=fake)
+    need = lib.af_attention_workspace_size(batch, 24, 8, 128, -(-rows // 512))
+    assert lib.af_paged_attention(fake, 3072, ctypes.byref(pool), 0, fake, 1000, fake, batch, rows,
+                                  fake, 3072, 24, 0, fake, need - 1,
+                                  None) == atomflow_amd.AF_ERR_WORKSPACE
+
+
 def test_missing_library_fails_loudly(monkeypatch):
     monkeypatch.setattr(atomflow_amd, "_lib", None)
     monkeypatch.setattr(atomflow_amd, "LIB_PATH", "/nonexistent/libatomflow_kv.so")
