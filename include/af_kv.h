@@ -234,7 +234,11 @@ int af_paged_rope_append(void* qkv_out, int batch, const af_kv_pool* pool, int l
  * batch <= 256, head_dim 128) with batch * max_seq_len >= 4096 rows per CU run
  * as one persistent launch whose workgroups claim row ranges from a counter in
  * the workspace (re-armed by the launch); small batches take splits whose spans
- * follow the sequence lengths, as many as the workspace holds records for. */
+ * follow the sequence lengths, as many as the workspace holds records for (the
+ * last bits then depend on the batch's other lengths and, below
+ * af_attention_workspace_size(batch, .., 0), on the workspace's size; an explicit
+ * num_splits keeps them independent). Both forms size themselves by max_seq_len: a
+ * bound far above the lengths costs a launch of short sequences time. */
 int af_paged_attention(const void* q, int q_stride, const af_kv_pool* pool, int layer,
                        const int32_t* d_block_tables, int max_blocks_per_seq,
                        const int32_t* d_seq_lens, int batch, int max_seq_len, void* out,
